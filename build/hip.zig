@@ -17,6 +17,7 @@ const Source = struct { file: []const u8, extra: []const []const u8 = &.{} };
 const sources = [_]Source{
     .{ .file = "attn_fwd.hip" },
     .{ .file = "attn_stream.hip", .extra = &.{ "-mllvm", "-pragma-unroll-threshold=1000000" } },
+    .{ .file = "attn_keysplit.hip", .extra = &.{ "-mllvm", "-pragma-unroll-threshold=1000000" } },
     .{ .file = "kv_image.hip" },
     .{ .file = "rms_rope.hip" },
     .{ .file = "int8_attn.hip" },

@@ -61,12 +61,17 @@ typedef struct ihipStream_t* lr_stream_t;
 #define LR_WEIGHT_F32 1
 #define LR_WEIGHT_BF16 2
 
-/* Attention tile configurations for the _ex entry points (0 = the library's choice: LR_ATTN_CFG_STREAM_W8 for the
- * fused and prepared calls; for attention over key and value rows, non-causal calls of at least 4,096 keys run
- * LR_ATTN_CFG_STREAM_W8 over the key rows when their 256-query blocks fill at least half a round of the device's
- * compute units without leaving a last round less than half full, or fill two rounds or more; other calls run
- * LR_ATTN_CFG_PIPE_W4, or LR_ATTN_CFG_PIPE_W8 when non-causal and the 256-query blocks fill whole rounds of the
- * compute units. The workspace call lr_attention_bf16_ws chooses as described there.) */
+/* Attention tile configurations for the _ex entry points. 0 = the library's choice by the call's sizes:
+ *   fused and prepared calls: LR_ATTN_CFG_STREAM_W8, or, non-causal with few 128-query blocks (at most one per compute
+ *     unit), the key-split kernel over the same tile images (attn_keysplit.hip: 128 queries per workgroup, two groups of
+ *     waves over alternating key tiles);
+ *   attention over key and value rows, from 449 keys on: the key-split kernel for causal calls and for non-causal ones
+ *     of at most one 128-query block per compute unit; else LR_ATTN_CFG_STREAM_W8 for non-causal calls of at least
+ *     4,096 keys whose 256-query blocks fill at least half a round of the device's compute units without leaving a last
+ *     round less than half full, or fill two rounds or more; other calls LR_ATTN_CFG_PIPE_W4, or LR_ATTN_CFG_PIPE_W8 when
+ *     non-causal and the 256-query blocks fill whole rounds of the compute units. The workspace call
+ *     lr_attention_bf16_ws chooses as described there.
+ */
 #define LR_ATTN_CFG_AUTO 0
 #define LR_ATTN_CFG_PIPE_W8 1      /* attention over value rows: 256 queries per workgroup (8 waves x 32), direct-to-LDS
                                       K/V ring, next tile's QK^T overlapped with the current tile's softmax */
@@ -111,8 +116,9 @@ int lr_attention_bf16_ex(const void* q, const void* k, const void* v, void* out,
 /*
  * lr_attention_bf16 with device scratch. A non-causal call with at most 32 blocks of 256 queries x heads and at least
  * 961 keys (16 tiles of 64; e.g. 218 queries over 50,220 keys) is split over the keys into ranges that fill the GPU,
- * each range's partial result written to the workspace, then merged (flash-decoding). Other non-causal calls of at least 4,096 keys
- * run LR_ATTN_CFG_STREAM_W8 over the key rows, whose last partial round of query blocks is cut over all workgroups
+ * each range's partial result written to the workspace, then merged (flash-decoding). Other non-causal calls of at least
+ * 4,096 keys (but for those of few query blocks whose keys the key-split kernel covers sooner) run
+ * LR_ATTN_CFG_STREAM_W8 over the key rows, whose last partial round of query blocks is cut over all workgroups
  * along the keys, the pieces' partials and arrival counters in the workspace (LR_JOINT_SPLIT_BYTES; the call clears
  * the counters itself). Every other call runs as lr_attention_bf16. lr_attention_ws_bytes is the workspace the call
  * needs (0: none; workspace may then be NULL); those bytes must not overlap q, k, v or out (rejected). Results equal

@@ -20,8 +20,8 @@ PKG = Path(__file__).resolve().parent
 ROOT = PKG.parent
 CSRC = PKG / "csrc"
 LIB = PKG / "liblr_attn.so"
-SOURCES = ["attn_fwd.hip", "attn_stream.hip", "kv_image.hip", "rms_rope.hip", "int8_attn.hip", "keys.hip", "lr_abi.hip",
-           "mmdit.hip", "rope_host.cpp"]
+SOURCES = ["attn_fwd.hip", "attn_stream.hip", "attn_keysplit.hip", "kv_image.hip", "rms_rope.hip", "int8_attn.hip",
+           "keys.hip", "lr_abi.hip", "mmdit.hip", "rope_host.cpp"]
 # libraries the shared object links: hipBLASLt for the MMDiT block's projections and MLP
 LIBS = ["-L/opt/rocm/lib", "-lhipblaslt"]
 ARCH = "gfx950"
@@ -40,7 +40,8 @@ HIPCC_FLAGS = [
 
 # per-source extra flags: the streaming kernel's fully unrolled key-tile step is larger than clang's default limit for
 # `#pragma unroll`, and a partly unrolled step would index its register arrays at run time
-EXTRA_FLAGS = {"attn_stream.hip": ["-mllvm", "-pragma-unroll-threshold=1000000"]}
+EXTRA_FLAGS = {"attn_stream.hip": ["-mllvm", "-pragma-unroll-threshold=1000000"],
+               "attn_keysplit.hip": ["-mllvm", "-pragma-unroll-threshold=1000000"]}
 
 # Scratch (spill) budget per kernel, bytes per lane. The streaming attention kernel and the INT8 attention kernel count
 # their direct global->LDS refills with explicit `s_waitcnt vmcnt(N)`; a scratch access among those loads would be

@@ -64,223 +64,7 @@ constexpr int PMAX = 4;                   // pieces a cut block is split into at
 constexpr int SLOT_WAVE_BYTES = 64 * 64 * 4 + 64 * 8;
 static_assert(SW * SLOT_WAVE_BYTES == STREAM_SLOT_BYTES, "partial slot size");
 
-// S = K Q^T with the accumulator starting at 0 / at c, and S += K Q^T: scores in VGPRs (the VALU reads them), Q in
-// AGPRs. Inline asm, so the compiler cannot move the 64 Q registers into VGPRs; every VALU read of a result below is
-// at least 16 MFMA slots after the MFMA, or behind a fence.
-__device__ __forceinline__ void qk_zero(f32x16& d, const bf16x8& k, const bf16x8& q) {
-    asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, 0" : "=&v"(d) : "v"(k), "a"(q));
-}
-__device__ __forceinline__ void qk_init(f32x16& d, const bf16x8& k, const bf16x8& q, const f32x16& c) {
-    asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %3" : "=&v"(d) : "v"(k), "a"(q), "v"(c));
-}
-__device__ __forceinline__ void qk_acc(f32x16& d, const bf16x8& k, const bf16x8& q) {
-    asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+v"(d) : "v"(k), "a"(q));
-}
-// O += V^T P: the builtin, so that the compiler knows it is an MFMA (O stays in AGPRs, hazards are its job)
-__device__ __forceinline__ void pv(f32x16& o, const bf16x8& v, const u32x4& p) {
-    o = __builtin_amdgcn_mfma_f32_32x32x16_bf16(v, __builtin_bit_cast(bf16x8, p), o, 0, 0, 0);
-}
-#define LR_NOP48 "s_nop 15\n\ts_nop 15\n\ts_nop 15"
-__device__ __forceinline__ void fence_s(f32x16& s) { asm volatile(LR_NOP48 : "+v"(s)); }
-__device__ __forceinline__ void fence_q8(bf16x8 (&q)[8]) {
-    asm volatile(LR_NOP48 : "+a"(q[0]), "+a"(q[1]), "+a"(q[2]), "+a"(q[3]), "+a"(q[4]), "+a"(q[5]), "+a"(q[6]),
-                 "+a"(q[7]));
-}
-
-// Two contiguous 1 KB direct loads, global -> LDS: lane l's 16 bytes of load i come from gaddr + 1024 i + 16 l and
-// land at LDS byte lds + 1024 i + 16 l (the instruction offset applies to both addresses).
-__device__ __forceinline__ void dma2k(uint64_t gaddr, uint32_t voff, uint32_t lds) {
-    LR_ASM_M0_BEGIN
-    asm volatile(
-        "s_mov_b32 m0, %2\n\t"
-        "s_nop 0\n\t"
-        "global_load_lds_dwordx4 %0, %1 offset:0\n\t"
-        "global_load_lds_dwordx4 %0, %1 offset:1024" ::"v"(voff),
-        "s"(gaddr), "s"(lds)
-        : "memory", "m0");
-    LR_ASM_M0_END
-}
-
-// Value tile rows in LDS: the 16 bytes of dims 8 c .. 8 c + 7 of tile row r (r < 64, c < 16) sit at byte
-// vt_offset(r, c) of the 16 KB slot: 4-row x 4-chunk blocks of 256 contiguous bytes, block (r >> 2, c >> 2) at
-// 256 (4 (r >> 2) + (c >> 2)), row r & 3 of it at + 64 (r & 3), chunk c & 3 at + 16 (c & 3). The address a lane reads
-// for value fragment (16-key step kk, 32-dim block db) is then additive: a per-lane part (VT_LANE) plus
-// 4096 kk + 256 db (+ 1024 for the fragment's second four keys), all immediates.
-__host__ __device__ constexpr int vt_offset(int r, int c) {
-    return 256 * (4 * (r >> 2) + (c >> 2)) + 64 * (r & 3) + 16 * (c & 3);
-}
-// Direct loads of a value tile: wave w's load i (i < 2) fills the slot's bytes 2048 w + 1024 i + 16 l (lane l), i.e.
-// rows 8 w + 4 i + vt_lane_row(l), chunk vt_lane_chunk(l) of the tile.
-__host__ __device__ constexpr int vt_lane_row(int l) { return (l >> 2) & 3; }
-__host__ __device__ constexpr int vt_lane_chunk(int l) { return 4 * (l >> 4) + (l & 3); }
-// The per-lane part of a transposed fragment read: lane l = 16 g + s reads (ds_read_b64_tr_b16: each group of 16
-// lanes takes a 4-row x 16-dim block, lane s pointing at row s >> 2, dims 4 (s & 3) .. +3, and gets dim s of the four
-// rows) keys 8 (l >> 5) + (s >> 2) of dims 16 (g & 1) + 4 (s & 3) .. of the fragment's 32-dim block.
-__host__ __device__ constexpr int vt_lane(int l) {
-    return 2048 * (l >> 5) + 64 * ((l >> 2) & 3) + 32 * ((l >> 4) & 1) + 8 * (l & 3);
-}
-
-// Two 1 KB direct loads of value rows, global -> LDS: lane l's 16 bytes of load 0 come from gaddr + voff0 and land at
-// LDS byte lds + 16 l; those of load 1 from gaddr + voff1 + 1024 to lds + 1024 + 16 l (the instruction offset applies
-// to both addresses; voff1 = voff0 + 4 rows - 1024 >= 0).
-__device__ __forceinline__ void dma2v(uint64_t gaddr, uint32_t voff0, uint32_t voff1, uint32_t lds) {
-    LR_ASM_M0_BEGIN
-    asm volatile(
-        "s_mov_b32 m0, %3\n\t"
-        "s_nop 0\n\t"
-        "global_load_lds_dwordx4 %0, %2 offset:0\n\t"
-        "global_load_lds_dwordx4 %1, %2 offset:1024" ::"v"(voff0),
-        "v"(voff1), "s"(gaddr), "s"(lds)
-        : "memory", "m0");
-    LR_ASM_M0_END
-}
-// The same two loads with their own M0 each and no instruction offset (the last, clamped tile of a head, whose
-// offsets may be smaller than 1024; and the key gathers of a call over key rows, whose lanes' offsets are rows apart).
-__device__ __forceinline__ void dma2_apart(uint64_t gaddr, uint32_t voff0, uint32_t voff1, uint32_t lds) {
-    LR_ASM_M0_BEGIN
-    asm volatile(
-        "s_mov_b32 m0, %3\n\t"
-        "s_nop 0\n\t"
-        "global_load_lds_dwordx4 %0, %2 offset:0\n\t"
-        "s_add_u32 m0, %3, 0x400\n\t"
-        "s_nop 0\n\t"
-        "global_load_lds_dwordx4 %1, %2 offset:0" ::"v"(voff0),
-        "v"(voff1), "s"(gaddr), "s"(lds)
-        : "memory", "m0", "scc");
-    LR_ASM_M0_END
-}
-// Key rows gathered into a tile image: lane l's 16 bytes of the two fragments a wave fills (at LDS byte lds + 16 l and
-// lds + 1024 + 16 l) are 8 dims of the same key row, 16 dims (32 bytes) apart: load 0 from gaddr + koff, load 1 from
-// gaddr + koff + 32 (its instruction offset 32 also adds to the LDS address, so M0 takes the other 992 bytes).
-__device__ __forceinline__ void dma2k_rows(uint64_t gaddr, uint32_t koff, uint32_t lds) {
-    LR_ASM_M0_BEGIN
-    asm volatile(
-        "s_mov_b32 m0, %2\n\t"
-        "s_nop 0\n\t"
-        "global_load_lds_dwordx4 %0, %1 offset:0\n\t"
-        "s_add_u32 m0, %2, 0x3e0\n\t"
-        "s_nop 0\n\t"
-        "global_load_lds_dwordx4 %0, %1 offset:32" ::"v"(koff),
-        "s"(gaddr), "s"(lds)
-        : "memory", "m0", "scc");
-    LR_ASM_M0_END
-}
-
-typedef __attribute__((address_space(3))) i16x4_t lds_i16x4;
-// One value fragment (the A operand V^T of O^T += V^T P^T: lane l = 32 hf + n gets keys 8 hf .. 8 hf + 7 of dim n of
-// the 16-key x 32-dim block) from the row-block LDS layout: addr = slot + VT_LANE + 4096 kk + 256 db.
-__device__ __forceinline__ bf16x8 vfrag_at(uint32_t addr) {
-    const i16x4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)(uintptr_t)addr);
-    const i16x4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)(uintptr_t)(addr + 1024));
-    return __builtin_shufflevector(__builtin_bit_cast(bf16x4, lo), __builtin_bit_cast(bf16x4, hi), 0, 1, 2, 3, 4, 5, 6,
-                                   7);
-}
-
-template <bool B>
-struct BoolTag {
-    static constexpr bool value = B;
-};
-template <int N>
-struct IntTag {
-    static constexpr int value = N;
-};
-
-typedef __attribute__((address_space(3))) const bf16x8 lds_frag;
-__device__ __forceinline__ bf16x8 frag_at(uint32_t addr) { return *(lds_frag*)(uintptr_t)addr; }
-
-// Recompute wave `wave`'s 32 queries of a block with the exact row maximum (the rare case of a non-finite row under the
-// fixed reference): pass 1 takes the maximum of every score, pass 2 accumulates P = exp2(S - max) <= 1, the row sums and
-// O, and the rows are written. The prepared queries are read from a.q (the block's rows, not yet overwritten), the key
-// fragments straight from the tile images in HBM (a 1 KB fragment is one 16-byte load per lane) or, KR, from the key
-// rows (lane 32 hf + n: 16 bytes of key 32 j + key_perm(n) for fragment ks, the tile image's content), and the value
-// fragments from the value rows (eight 2-byte loads per lane): nothing here touches LDS or waits for the other waves.
-// Called after the streaming loop, so that its registers do not add to the loop's.
-template <bool KR>
-__device__ __forceinline__ void redo_exact(const AttnArgs& a, int head, int hk, int row0, int tiles, int wave) {
-    const int lane = threadIdx.x & 63, n = lane & 31, hf = lane >> 5;
-    const int wrow0 = row0 + wave * 32, qrow = wrow0 + n;
-    const int T = (a.nkeys + IMG_TILE_KEYS - 1) / IMG_TILE_KEYS;
-    const uint64_t head_off = (uint64_t)hk * T * IMG_TILE_BYTES + (uint64_t)lane * 16;
-    const uint8_t* kh = reinterpret_cast<const uint8_t*>(a.k) + head_off;
-    const uint16_t* krows = a.k + (int64_t)hk * a.k_hs + 8 * hf;
-    const uint16_t* vh = a.v + (int64_t)hk * a.v_hs + n;   // dim n of this lane's 32-dim blocks
-    bf16x8 qf[8];
-    const uint16_t* src = a.q + (int64_t)min(qrow, a.W - 1) * a.q_rs + head * D + 8 * hf;
-#pragma unroll
-    for (int ks = 0; ks < 8; ++ks) qf[ks] = *reinterpret_cast<const bf16x8*>(src + 16 * ks);
-    int lim0 = a.nkeys;
-    if (a.causal) lim0 = min(lim0, a.p0 + qrow + 1);
-    auto scores = [&](int j, const f32x16& c) {
-        const uint8_t* kt = kh + (uint64_t)(j >> 1) * IMG_TILE_BYTES + (j & 1) * 8 * IMG_FRAG_BYTES;
-        // KR: keys past nkeys read the last row (finite; masked below)
-        const uint16_t* kr = krows + (int64_t)min(32 * j + img_key_perm(n), a.nkeys - 1) * a.k_rs;
-        f32x16 sr = c;
-#pragma unroll
-        for (int ks = 0; ks < 8; ++ks) {
-            const bf16x8 kf = KR ? *reinterpret_cast<const bf16x8*>(kr + 16 * ks)
-                                 : *reinterpret_cast<const bf16x8*>(kt + ks * IMG_FRAG_BYTES);
-            sr = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf, qf[ks], sr, 0, 0, 0);
-        }
-        const int lim = lim0 - (32 * j + 8 * hf);
-#pragma unroll
-        for (int r = 0; r < 16; ++r)
-            if (!(16 * (r >> 3) + (r & 7) < lim)) sr[r] = -INFINITY;
-        return sr;
-    };
-    float mx = -INFINITY;
-    for (int j = 0; j < 2 * tiles; ++j) {
-        const f32x16 sr = scores(j, f32x16{});
-#pragma unroll
-        for (int r = 0; r < 16; ++r) mx = fmaxf(mx, sr[r]);
-    }
-    const float m = wave_pair_max(mx);
-    const f32x16 nm = f32x16{} - (m > -INFINITY ? m : 0.0f);
-    const float c = a.c;
-    f32x16 o[4] = {};
-    float ls = 0.0f;
-    for (int j = 0; j < 2 * tiles; ++j) {
-        const f32x16 sr = scores(j, nm);
-        // value fragment x of the half-tile (16-key step x >> 2, 32-dim block x & 3): keys 32 j + 16 (x >> 2) +
-        // 8 hf .. +7 of dim 32 (x & 3) + n, eight 2-byte loads (rows past nkeys read the last row: their P is 0)
-        auto vfrag = [&](int x) {
-            uint16_t e[8];
-#pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                const int key = min(32 * j + 16 * (x >> 2) + 8 * hf + i, a.nkeys - 1);
-                e[i] = vh[(int64_t)key * a.v_rs + 32 * (x & 3)];
-            }
-            u32x4 w;
-#pragma unroll
-            for (int i = 0; i < 4; ++i) w[i] = (uint32_t)e[2 * i] | ((uint32_t)e[2 * i + 1] << 16);
-            return __builtin_bit_cast(bf16x8, w);
-        };
-        u32x4 pr[2];
-#pragma unroll
-        for (int w = 0; w < 8; ++w) {
-            const float e0 = __builtin_amdgcn_exp2f(sr[8 * (w >> 2) + 2 * (w & 3)] * c);
-            const float e1 = __builtin_amdgcn_exp2f(sr[8 * (w >> 2) + 2 * (w & 3) + 1] * c);
-            pr[w >> 2][w & 3] = pack_bf16x2(e0, e1);
-            ls += e0 + e1;
-        }
-#pragma unroll
-        for (int x = 0; x < 8; ++x)
-            o[x & 3] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vfrag(x), __builtin_bit_cast(bf16x8, pr[x >> 2]),
-                                                            o[x & 3], 0, 0, 0);
-    }
-    const float inv = 1.0f / wave_pair_sum(ls);
-    if (qrow < a.W) {
-        uint16_t* dst = a.out + (int64_t)qrow * a.o_rs + head * D + 4 * hf;
-#pragma unroll
-        for (int db = 0; db < 4; ++db)
-#pragma unroll
-            for (int gg = 0; gg < 4; ++gg) {
-                u32x2 w;
-                w[0] = pack_bf16x2(o[db][4 * gg] * inv, o[db][4 * gg + 1] * inv);
-                w[1] = pack_bf16x2(o[db][4 * gg + 2] * inv, o[db][4 * gg + 3] * inv);
-                *reinterpret_cast<u32x2*>(dst + 32 * db + 8 * gg) = w;
-            }
-    }
-}
+#include "attn_tiles.inc"
 
 // KR: a.k holds key rows (key j of kv head g at a.k + g * a.k_hs + j * a.k_rs), gathered into the tile-image layout by
 // the ring's direct loads; otherwise a.k holds the tile images.

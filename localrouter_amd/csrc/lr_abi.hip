@@ -76,6 +76,34 @@ bool stream_rows_split(int W, int H, int nkeys, int cus) {
     return !(nkeys > 16384 && 4 * tail >= 3 * (int64_t)cus);
 }
 
+// Whether a non-causal call runs the key-split kernel (attn_keysplit.hip: 128-query blocks, one workgroup each, two key
+// groups) in place of the streaming kernel (or, over rows, the pipelined kernels): its blocks fit one round of the CUs
+// and, where the streaming kernel could cut its tail (split_area), half the key tiles are no more than the tiles a
+// workgroup of that tail takes plus 12 (the ~16 us its partials, merges and longer start cost, at ~1.3 us a tile).
+// Measured (us, this kernel / the other): fused 320 x 4 heads 14.9 / 24.5, 512 x 24 18.8 / 30.9, 1,280 x 24 34.3 / 48.4,
+// 3,000 x 4 43.0 / 50.1; past one round it gains nothing (fused 1,600 x 24, 1.2 rounds, 59.9 / 60.5; 3,000 x 12, 1.1
+// rounds, 90.8 / 77.5; 4,608 x 24 263 / 248); over rows against the 128-query pipelined kernel 600 x 16 14.9 / 16.5,
+// 1,024 queries x 1,104 keys x 32 23.6 / 26.5, 1,280 x 24 26.1 / 27.2, and 2,000 x 24 (1.5 rounds) 69.6 / 60.3.
+bool keysplit_fits(int W, int H, int nkeys, int cus, bool split_area) {
+    const int64_t blocks = (int64_t)((W + 127) / 128) * H, T = (nkeys + 63) / 64;
+    if (blocks > cus) return false;
+    int tail_wg = 0;
+    const int nwg = std::min(cus, lr::STREAM_MAX_WG);
+    if (!split_area || !lr::stream_split_params(W, H, nkeys, 0, nwg, &tail_wg)) return true;
+    const int64_t tail = (int64_t)((W + 255) / 256) * H % nwg;   // <= blocks <= cus: all of them when below nwg
+    return (T + 1) / 2 <= (tail * T + tail_wg - 1) / tail_wg + 12;
+}
+
+// The same over key and value rows. The pipelined kernel starts sooner (~2.5 us: fewer loads before its first product, no
+// merge), so calls of fewer than 8 key tiles keep it (320 x 4 heads 11.7 / 10.4 us, 256 x 24 10.6 / 9.8). Causal calls
+// take the key-split kernel whatever their size: its blocks run longest first and each in half the steps (1,500 queries
+// x 1,577 keys, 32 heads over 8, 32.7 / 40.4 us; 2,048 42.7 / 57.8; 4,096 140 / 187; 4,608 x 24 142 / 178).
+bool keysplit_rows(int W, int H, int nkeys, int causal, int cus, bool split_area) {
+    if (nkeys <= 7 * 64 || cus < 1) return false;
+    if ((int64_t)((W + 127) / 128) * H > 1 << 22) return false;   // (a grid's work-items are counted in 32 bits)
+    return causal || keysplit_fits(W, H, nkeys, cus, split_area);
+}
+
 size_t split_bytes(int W, int H, int ns) {
     if (ns <= 1) return 0;
     const size_t rows = (size_t)H * W * ns;
@@ -117,14 +145,18 @@ int attention_impl(const void* q, const void* k, const void* v, void* out, int p
         return (int)lr::launch_split_combine(a, stream);
     }
     const bool ws_split_area = workspace && ws_bytes >= (size_t)LR_JOINT_SPLIT_BYTES && aligned(workspace, 256);
-    if (config == LR_ATTN_CFG_AUTO && stream_rows(W, H, nkeys, causal, ws_split_area, device_cus())) {
+    // (the key-split kernel takes 32-bit per-lane row offsets, as the streaming kernel does: wider strides go on)
+    const int cus = config == LR_ATTN_CFG_AUTO || config == LR_ATTN_CFG_STREAM_W8 ? device_cus() : 0;
+    if (config == LR_ATTN_CFG_AUTO && keysplit_rows(W, H, nkeys, causal, cus, ws_split_area) &&
+        k_rs <= lr::STREAM_MAX_V_RS && v_rs <= lr::STREAM_MAX_V_RS)
+        return (int)lr::launch_keysplit(a, stream, true);
+    if (config == LR_ATTN_CFG_AUTO && stream_rows(W, H, nkeys, causal, ws_split_area, cus)) {
         config = LR_ATTN_CFG_STREAM_W8;
     } else if (config == LR_ATTN_CFG_AUTO) {
         // 128 queries per workgroup, two workgroups per CU, unless non-causal 256-query blocks fill whole rounds of
         // the CUs: measured at cfg1 / cfg2 / causal GQA shapes W4 takes 0.72 / 0.93 / 0.89 of W8's time, at 12,800
         // and 50,220 tokens the two are within 1.5 %, at 16,384 x 4 heads (exactly one round of 256-query blocks) W8
         // is 2 % faster; causal blocks differ in work, and W4 stays faster there even when the rounds are whole
-        const int cus = device_cus();
         const int64_t w8_blocks = (int64_t)((W + 255) / 256) * H;
         config = !causal && cus > 0 && w8_blocks % cus == 0 ? LR_ATTN_CFG_PIPE_W8 : LR_ATTN_CFG_PIPE_W4;
     }
@@ -132,13 +164,13 @@ int attention_impl(const void* q, const void* k, const void* v, void* out, int p
         // the streaming kernel over the key rows: the output's 32-bit buffer range (256 rows * o_rs * 2 bytes < 2^32)
         // and 32-bit per-lane row offsets (k_rs, v_rs <= STREAM_MAX_V_RS); with a workspace, its split tail
         if (o_rs >= ((int64_t)1 << 23) || k_rs > lr::STREAM_MAX_V_RS || v_rs > lr::STREAM_MAX_V_RS) return ERR_ARGS;
-        const int cus = std::min(device_cus(), lr::STREAM_MAX_WG);
-        if (cus < 1) return (int)hipErrorInvalidDevice;
-        if (ws_split_area && stream_rows_split(W, H, nkeys, cus)) {
+        const int nwg = std::min(cus, lr::STREAM_MAX_WG);
+        if (nwg < 1) return (int)hipErrorInvalidDevice;
+        if (ws_split_area && stream_rows_split(W, H, nkeys, nwg)) {
             a.part = workspace;
             a.cnt = reinterpret_cast<int*>(static_cast<char*>(workspace) + lr::STREAM_PART_BYTES);
         }
-        return (int)lr::launch_stream(a, cus, stream, true);
+        return (int)lr::launch_stream(a, nwg, stream, true);
     }
     return (int)lr::launch_attention(a, config, stream);
 }
@@ -323,7 +355,7 @@ bool images_stage_ok(const void* q_prep, int64_t p_rs, const void* ws, size_t ws
 // workspace's split area). v / v_rs: the value rows it reads (the caller's, or null for the workspace's value area).
 int images_launch(const void* q_prep, int64_t p_rs, const void* ws, void* out, int64_t o_rs, int Sq, int Sk, int H,
                   int HK, int p0, int causal, float scale, hipStream_t stream, const void* v = nullptr,
-                  int64_t v_rs = 0) {
+                  int64_t v_rs = 0, int config = LR_ATTN_CFG_AUTO) {
     const int cus = std::min(device_cus(), lr::STREAM_MAX_WG);
     if (cus < 1) return (int)hipErrorInvalidDevice;
     lr::AttnArgs a{};
@@ -345,6 +377,8 @@ int images_launch(const void* q_prep, int64_t p_rs, const void* ws, void* out, i
     char* split = split_area(const_cast<void*>(ws), Sk, HK);
     a.part = split;
     a.cnt = reinterpret_cast<int*>(split + lr::STREAM_PART_BYTES);
+    if (config == LR_ATTN_CFG_AUTO && !causal && keysplit_fits(Sq, H, Sk, cus, true))
+        return (int)lr::launch_keysplit(a, stream, false);
     return (int)lr::launch_stream(a, cus, stream);
 }
 
@@ -361,7 +395,7 @@ int prepared_impl(const void* q_raw, void* ws, size_t ws_bytes, void* out, const
     const int e = q_launch(q_raw, q_rs, out, o_rs, wq, table_kind, qta, qtb, tab_stride, pairing, rot, eps, Sq, H,
                            stream);
     if (e != 0) return e;
-    return images_launch(out, o_rs, ws, out, o_rs, Sq, Sk, H, HK, p0, causal, scale, stream);
+    return images_launch(out, o_rs, ws, out, o_rs, Sq, Sk, H, HK, p0, causal, scale, stream, nullptr, 0, config);
 }
 
 int fused_impl(const void* q_raw, const void* k_raw, const void* v, void* out, const float* wq, const float* wk,
@@ -385,7 +419,7 @@ int fused_impl(const void* q_raw, const void* k_raw, const void* v, void* out, c
     const int e = prep_launch(q_raw, q_rs, out, o_rs, wq, k_raw, k_rs, v, v_rs, wk, table_kind, qta, qtb, kta, ktb,
                               tab_stride, pairing, rot, eps, Sq, Sk, H, HK, n_pre, ws, 0, stream);
     if (e != 0) return e;
-    return images_launch(out, o_rs, ws, out, o_rs, Sq, Sk, H, HK, p0, causal, scale, stream, v, v_rs);
+    return images_launch(out, o_rs, ws, out, o_rs, Sq, Sk, H, HK, p0, causal, scale, stream, v, v_rs, config);
 }
 
 int rope_impl(const void* src, int64_t src_rs, int64_t src_off, void* dst, int64_t dst_rs, int64_t n, int b,

@@ -103,6 +103,11 @@ hipError_t launch_joint_prep(const KvImageArgs& kv, const RopeArgs& q, hipStream
 // a.part / a.cnt: the partial area and arrival counters of the workspace (null: whole blocks only); nwg <=
 // STREAM_MAX_WG.
 hipError_t launch_stream(const AttnArgs& a, int nwg, hipStream_t stream, bool key_rows = false);
+// Whether launch_stream cuts the last partial round of a call's blocks over workgroups, and over how many.
+bool stream_split_params(int W, int H, int nkeys, int causal, int nwg, int* tail_wg);
+// The same contract as launch_stream without a split area, for calls of few query blocks (attn_keysplit.hip): 128-query
+// blocks, one workgroup each, its waves cut over the keys.
+hipError_t launch_keysplit(const AttnArgs& a, hipStream_t stream, bool key_rows = false);
 constexpr int64_t STREAM_MAX_V_RS = (int64_t)1 << 24;                   // value row stride (elements) at most
 constexpr int STREAM_MAX_WG = 256;                                      // workgroups of one streaming launch at most
 constexpr int64_t STREAM_SLOT_BYTES = 8 * (64 * 64 * 4 + 64 * 8);        // one piece's partial: 8 waves' O, m and l
