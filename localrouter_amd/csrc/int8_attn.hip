@@ -736,9 +736,10 @@ constexpr float LAZY = 64.0f;
 //   A: S(t+1) = K(t+1) Q^T (int8 MFMA, two 32-key accumulator chains alternating), and in the same slots P(t) from
 //      S(t): x = s * c - m_t (one FMA on the biased score), P = exp2(x) to u8, its row sum (udot4), P ^ 0x80;
 //   B: O^T += V(t)^T P(t) (int8 MFMA, one 32-dim block after the other, two accumulators alternating), and in the
-//      same slots the fp32 update of the previous block, O += ts * acc, and the row max of S(t+1);
+//      same slots the fp32 update of the previous block, O += ts * acc, the row max of S(t+1) and then tile t+1's
+//      constants (max, scales);
 //   operand fragments are read from LDS two slots ahead;
-//   then the column-sum correction (one f32 MFMA per 32-dim block) and tile t+1's constants (max, scales).
+//   then the column-sum correction (one f32 MFMA per 32-dim block).
 // K, V^T and the aux block of tile t+3 are loaded into a 4-stage LDS ring while tiles t and t+1 are read.
 // A workgroup below a.nwhole computes one query block over all key tiles and writes its rows; one at or past it (a
 // piece) computes a block of the last partial round over its key range [t0, t1) and leaves the unnormalised rows and
@@ -761,7 +762,7 @@ __global__ __launch_bounds__(512, 1) __attribute__((amdgpu_waves_per_eu(2, 2))) 
     __shared__ __attribute__((aligned(1024))) uint8_t ring[NS * STAGE];
 
     const Plan& p = a.p;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int n = lane & 31, hf = lane >> 5;
 
     // Whole blocks (workgroups below nwhole) in XCD-aware order: consecutive logical blocks (same head) land on the
@@ -821,32 +822,31 @@ __global__ __launch_bounds__(512, 1) __attribute__((amdgpu_waves_per_eu(2, 2))) 
 
     // ring stage of tile t (a piece's first tile t0 is a multiple of NS: its ring starts at stage 0 too)
     auto stage = [&](int t) { return ring + (t % NS) * STAGE; };
-    auto issue = [&](int t) {
-        uint8_t* st = stage(t);
+    // load i < LPT of tile t
+    auto issue1 = [&](int t, uint8_t* st, int i) {
         if constexpr (KVL > 0) {
-#pragma unroll
-            for (int i = 0; i < KVL; ++i) {
-                const int blk = wave * KVL + i;
-                dma16(k8 + (size_t)t * TB + blk * 1024, lane * 16, lds_addr(st + blk * 1024));
-                dma16(vt + (size_t)t * TB + blk * 1024, lane * 16, lds_addr(st + TB + blk * 1024));
-            }
-        } else if (wave < NBLK) {
-            dma16(k8 + (size_t)t * TB + wave * 1024, lane * 16, lds_addr(st + wave * 1024));
+            const int blk = wave * KVL + (i >> 1);
+            if (i & 1) dma16(vt + (size_t)t * TB + blk * 1024, lane * 16, lds_addr(st + TB + blk * 1024));
+            else dma16(k8 + (size_t)t * TB + blk * 1024, lane * 16, lds_addr(st + blk * 1024));
         } else {
-            dma16(vt + (size_t)t * TB + (wave - NBLK) * 1024, lane * 16, lds_addr(st + TB + (wave - NBLK) * 1024));
+            const bool kw = wave < NBLK;
+            const size_t off = (size_t)t * TB + (kw ? wave : wave - NBLK) * 1024;
+            dma16((kw ? k8 : vt) + off, lane * 16, lds_addr(st + wave * 1024));
         }
+    };
+    // wave 0 loads the aux block too
+    auto issue_aux = [&](int t, uint8_t* st) {
         if (wave == 0) dma16(aux + (size_t)t * AUX_BYTES, lane * 16, lds_addr(st + 2 * TB));
     };
-    // wait until tile `need` has landed, given that tiles up to `issued` were issued
-    auto wait_for = [&](int need, int issued) {
-        const bool one = issued > need;  // at most one later tile (NS = 4: issued <= need + 1)
-        if (wave == 0) {
-            if (one) LR_I8_WAIT_VMCNT(LPT + 1);
-            else LR_I8_WAIT_VMCNT(0);
-        } else {
-            if (one) LR_I8_WAIT_VMCNT(LPT);
-            else LR_I8_WAIT_VMCNT(0);
-        }
+    auto issue = [&](int t) {
+        issue_aux(t, stage(t));
+#pragma unroll
+        for (int i = 0; i < LPT; ++i) issue1(t, stage(t), i);
+    };
+    // wait until this wave's loads of all tiles but the last one issued have landed
+    auto wait_but_last = [&]() {
+        if (wave == 0) LR_I8_WAIT_VMCNT(LPT + 1);
+        else LR_I8_WAIT_VMCNT(LPT);
     };
 
     i32x16 magic;
@@ -867,6 +867,10 @@ __global__ __launch_bounds__(512, 1) __attribute__((amdgpu_waves_per_eu(2, 2))) 
     // weight ts = 2^(m_t - m_run) <= 2^LAZY, so O stays below 2^64 * 255 * 127 * cta * ntiles (far from the fp32
     // range) and the rescale of O, which a running maximum would need on most tiles, is rare. O / l is the same
     // softmax: every tile's weight relative to any fixed reference cancels in the quotient.
+    // (For the first tile; the others' are computed by step t - 1 in the second half of its phase B, the same arithmetic
+    // spread over the slots: as one block after the phase, a chain of ~60 dependent instructions, it held both waves of a
+    // SIMD up at the same time. With the refills spread: 5,967 tokens x 56 heads 725 -> 704 us, at head dim 64 670 -> 627,
+    // 1,797 x 32 x 64 43.8 -> 41.4, bit-identical.)
     auto constants = [&](const int (&mi)[NB], const uint8_t* st) {
         const uint8_t* ksp = st + 2 * TB + AUX_KS_OFF + 4 * NB * hf;
         float tmx = -INFINITY;
@@ -903,7 +907,8 @@ __global__ __launch_bounds__(512, 1) __attribute__((amdgpu_waves_per_eu(2, 2))) 
 #pragma unroll
     for (int j = 0; j < NS - 1; ++j)
         if (t0 + j < t1) issue(t0 + j);
-    wait_for(1, min(NS - 2, t1 - t0 - 1));
+    if (t0 + NS - 1 <= t1) wait_but_last();   // tiles t0 and t0 + 1
+    else LR_I8_WAIT_VMCNT(0);
     block_barrier();
     i32x16 SS[2][NB];  // S(t) in SS[t & 1]
     {
@@ -928,7 +933,11 @@ __global__ __launch_bounds__(512, 1) __attribute__((amdgpu_waves_per_eu(2, 2))) 
         constexpr bool LAST = decltype(last_c)::value;
         i32x16 (&S)[NB] = SS[PAR];
         i32x16 (&Sn)[NB] = SS[PAR ^ 1];
-        if (t + NS - 1 < t1) issue(t + NS - 1);
+        // tile t + NS - 1 into the stage tile t - 1 left, its loads spread over phase A (all at its start they held the
+        // waves' issue up behind the memory pipe); past the last tile a repeat of it, never read
+        const int tr = min(t + NS - 1, t1 - 1);
+        uint8_t* stR = stage(t + NS - 1);
+        if (NEXT) issue_aux(tr, stR);
         const uint8_t* stK = stage(t + 1);
         const uint8_t* stV = stage(t);
         const bool mask_p = LAST && t1 == ntiles && tail < CTA;
@@ -944,6 +953,7 @@ __global__ __launch_bounds__(512, 1) __attribute__((amdgpu_waves_per_eu(2, 2))) 
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int s = 0; s < 4 * NB; ++s) {
+            if (NEXT && s % (4 * NB / LPT) == 0) issue1(tr, stR, s / (4 * NB / LPT));
             if (NEXT && s % SPM == 0) {  // score MFMA f in the first slot of its group of SPM
                 const int f = s / SPM;
                 if (f + 2 < QS) fr[(f + 2) % 3] = kfrag(stK, f + 2);
@@ -976,6 +986,11 @@ __global__ __launch_bounds__(512, 1) __attribute__((amdgpu_waves_per_eu(2, 2))) 
         int mi[NB];
 #pragma unroll
         for (int kb = 0; kb < NB; ++kb) mi[kb] = MAGIC - (1 << 22);
+        float ksv[NB], tmx = -INFINITY, m_new = m_run, os = 1.0f, ts_next = ts;
+        if (NEXT) {
+#pragma unroll
+            for (int kb = 0; kb < NB; ++kb) ksv[kb] = lds_load<float>(stK + 2 * TB + AUX_KS_OFF + 4 * NB * hf + 4 * kb);
+        }
         i32x16 acc[2];
         fr[0] = vfrag(stV, 0);
         fr[1] = vfrag(stV, 1);
@@ -986,13 +1001,34 @@ __global__ __launch_bounds__(512, 1) __attribute__((amdgpu_waves_per_eu(2, 2))) 
             const int bb = s / NB, j = s % NB;
             const i32x4 B = {(int)P[j][0], (int)P[j][1], (int)P[j][2], (int)P[j][3]};
             acc[bb & 1] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fr[s % 3], B, j == 0 ? magic : acc[bb & 1], 0, 0, 0);
-            if (NEXT) {  // max of S(t+1): its NB * 16 registers spread evenly over the PS slots
-                static_assert(NB * 16 % (4 * PS) == 0, "whole groups of 4 registers per slot");
+            if (NEXT) {
+                // the max of S(t+1), its registers over the first half of the slots, then tile t+1's constants
+                constexpr int RPS = NB * 16 / (PS / 2);
+                static_assert(RPS % 4 == 0, "whole groups of 4 registers per slot");
+                if (s < PS / 2) {
 #pragma unroll
-                for (int u = 0; u < NB * 16 / PS / 4; ++u) {
-                    const int g = (NB * 16 / PS) * s + 4 * u;  // flat register index kb * 16 + r, < NB * 16
-                    const int kb = g >> 4, r = g & 15;
-                    mi[kb] = max(max(mi[kb], Sn[kb][r]), max(max(Sn[kb][r + 1], Sn[kb][r + 2]), Sn[kb][r + 3]));
+                    for (int u = 0; u < RPS / 4; ++u) {
+                        const int g = RPS * s + 4 * u;  // flat register index kb * 16 + r, < NB * 16
+                        const int kb = g >> 4, r = g & 15;
+                        mi[kb] = max(max(mi[kb], Sn[kb][r]), max(max(Sn[kb][r + 1], Sn[kb][r + 2]), Sn[kb][r + 3]));
+                    }
+                }
+                if (s == PS / 2) {
+#pragma unroll
+                    for (int kb = 0; kb < NB; ++kb) {
+                        cc[kb] = cq * ksv[kb];
+                        tmx = fmaxf(tmx, (__int_as_float(mi[kb]) - MAGF) * cc[kb]);
+                    }
+                }
+                if (s == PS * 5 / 8) {
+                    tmx = pair_max(tmx) - S_U8_OFFSET;
+                    m_new = tmx > m_run + LAZY ? tmx : m_run;
+                }
+                if (s == PS * 3 / 4) {
+                    os = __builtin_amdgcn_exp2f(m_run - m_new);
+                    ts_next = __builtin_amdgcn_exp2f(tmx - m_new);
+#pragma unroll
+                    for (int kb = 0; kb < NB; ++kb) nbias[kb] = -fmaf(MAGF, cc[kb], tmx);
                 }
             }
             if (bb >= 1) {  // fp32 update of block bb - 1, spread over block bb's slots
@@ -1008,7 +1044,9 @@ __global__ __launch_bounds__(512, 1) __attribute__((amdgpu_waves_per_eu(2, 2))) 
 #pragma unroll
         for (int r = 0; r < 16; ++r) O[DB - 1][r] = fmaf(__int_as_float(acc[(DB - 1) & 1][r]), ts, O[DB - 1][r]);
         {
-            // + 128 * ts * (column sums of V(t)) - 12582912 * ts (the P V accumulator bias), per 32-dim block
+            // + 128 * ts * (column sums of V(t)) - 12582912 * ts (the P V accumulator bias), per 32-dim block (moved into
+            // the next tile's phase A, where the matrix cores have idle slots on paper, it was slower: 640 against 627 us
+            // at head dim 64, and spills at 128)
             int16_t cs[DB];
             if constexpr (DB == 4) {
                 const i16x4 c4 = lds_load<i16x4>(stV + 2 * TB + 8 * lane);
@@ -1025,9 +1063,16 @@ __global__ __launch_bounds__(512, 1) __attribute__((amdgpu_waves_per_eu(2, 2))) 
                 O[bb] = __builtin_amdgcn_mfma_f32_32x32x2f32((float)cs[bb] - 49152.0f, w128, O[bb], 0, 0, 0);
         }
         if (NEXT) {
-            constants(mi, stK);
-            if (t + 2 < t1) wait_for(t + 2, min(t1 - 1, t + NS - 1));
-            else LR_I8_WAIT_VMCNT(0);
+            ts = ts_next;
+            m_run = m_new;
+            if (__builtin_amdgcn_ballot_w64(os != 1.0f) != 0) {
+                l_run *= os;
+#pragma unroll
+                for (int bb = 0; bb < DB; ++bb)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) O[bb][r] *= os;
+            }
+            wait_but_last();   // tile t + 2 has landed
             block_barrier();
         }
     };
@@ -1046,6 +1091,7 @@ __global__ __launch_bounds__(512, 1) __attribute__((amdgpu_waves_per_eu(2, 2))) 
         step(t, P0{}, std::false_type{}, std::true_type{});
     }
 
+    LR_I8_WAIT_VMCNT(0);   // no direct load is still writing LDS when the workgroup ends
     if (!qok) return;
     const float* vs = reinterpret_cast<const float*>(a.ws + p.vs) + bhk * HD;
     if (piece) {   // the piece's unnormalised rows times the V scales, and (reference, row sum), to the partial area
