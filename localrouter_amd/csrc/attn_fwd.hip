@@ -56,7 +56,7 @@ __global__ __launch_bounds__(NW * 64, 8 / NW) __attribute__((amdgpu_waves_per_eu
     __shared__ __attribute__((aligned(1024))) uint16_t Kr[NS * TILE];
     __shared__ __attribute__((aligned(1024))) uint16_t Vr[NS * TILE];
 
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int n = lane & 31, hf = lane >> 5;
 
     const int nwg = gridDim.x, b = blockIdx.x;
@@ -96,54 +96,53 @@ __global__ __launch_bounds__(NW * 64, 8 / NW) __attribute__((amdgpu_waves_per_eu
     }
     const int vcol = 8 * (lchunk ^ (lrow << 2));   // rows 4i + lrow: (r & 3) == lrow
     const uint32_t kr_lds = lds_addr(Kr), vr_lds = lds_addr(Vr);
-    // Source pointers of the next K and V tiles to load, advanced one tile per issue; a tile reaching past nkeys
-    // takes the clamped path instead.
+    // Source pointers of the next K and V tiles to load. next_k / next_v move them to tile t before its loads: one tile
+    // on, or, in a tile reaching past nkeys, to the clamped rows.
     const int64_t kstep = (int64_t)BT * a.k_rs, vstep = (int64_t)BT * a.v_rs;
     const uint16_t* kp[LOADS];
     const uint16_t* vp[LOADS];
 #pragma unroll
     for (int j = 0; j < LOADS; ++j) {
-        kp[j] = kbase + (int64_t)krow[j] * a.k_rs + kcol[j];
-        vp[j] = vbase + (int64_t)krow[j] * a.v_rs + vcol;
+        kp[j] = kbase + ((int64_t)krow[j] - BT) * a.k_rs + kcol[j];
+        vp[j] = vbase + ((int64_t)krow[j] - BT) * a.v_rs + vcol;
     }
-    auto issue_k = [&](int t, int slot) {
-        const int key0 = t * BT;
-        const uint32_t dst = kr_lds + 2 * (slot * TILE + wave * 512);
-        if (key0 + BT <= a.nkeys) {
+    auto next_k = [&](int t) {
+        if ((t + 1) * BT <= a.nkeys) {
 #pragma unroll
-            for (int j = 0; j < LOADS; ++j) dma16(kp[j], dst + 2 * NW * 512 * j);
+            for (int j = 0; j < LOADS; ++j) kp[j] += kstep;
         } else {
 #pragma unroll
-            for (int j = 0; j < LOADS; ++j) {
-                const int key = min(key0 + krow[j], a.nkeys - 1);
-                dma16(kbase + (int64_t)key * a.k_rs + kcol[j], dst + 2 * NW * 512 * j);
-            }
+            for (int j = 0; j < LOADS; ++j)
+                kp[j] = kbase + (int64_t)min(t * BT + krow[j], a.nkeys - 1) * a.k_rs + kcol[j];
         }
-#pragma unroll
-        for (int j = 0; j < LOADS; ++j) kp[j] += kstep;
     };
-    auto issue_v = [&](int t, int slot) {
-        const int key0 = t * BT;
-        const uint32_t dst = vr_lds + 2 * (slot * TILE + wave * 512);
-        if (key0 + BT <= a.nkeys) {
+    auto next_v = [&](int t) {
+        if ((t + 1) * BT <= a.nkeys) {
 #pragma unroll
-            for (int j = 0; j < LOADS; ++j) dma16(vp[j], dst + 2 * NW * 512 * j);
+            for (int j = 0; j < LOADS; ++j) vp[j] += vstep;
         } else {
 #pragma unroll
-            for (int j = 0; j < LOADS; ++j) {
-                const int key = min(key0 + krow[j], a.nkeys - 1);
-                dma16(vbase + (int64_t)key * a.v_rs + vcol, dst + 2 * NW * 512 * j);
-            }
+            for (int j = 0; j < LOADS; ++j)
+                vp[j] = vbase + (int64_t)min(t * BT + krow[j], a.nkeys - 1) * a.v_rs + vcol;
         }
-#pragma unroll
-        for (int j = 0; j < LOADS; ++j) vp[j] += vstep;
     };
+    const uint32_t wdst = 2 * 512 * (uint32_t)__builtin_amdgcn_readfirstlane(wave);
+    auto load_k1 = [&](int slot, int j) { dma16(kp[j], kr_lds + 2 * slot * TILE + wdst + 2 * NW * 512 * j); };
+    auto load_v1 = [&](int slot, int j) { dma16(vp[j], vr_lds + 2 * slot * TILE + wdst + 2 * NW * 512 * j); };
 
     // ---- queries (B operands of S^T = K Q^T), one set per 32-query block
     // ---- prologue loads: K(0 .. NS-1) and V(0 .. NS-2) into the ring first, so that their latency overlaps the
     // query loads (the query's own waits, issued after, are conservative for the ring loads: older loads finish first)
-    for (int i = 0; i < NS && i < ntiles; ++i) issue_k(i, i);
-    for (int i = 0; i < NS - 1 && i < ntiles; ++i) issue_v(i, i);
+    for (int i = 0; i < NS && i < ntiles; ++i) {
+        next_k(i);
+#pragma unroll
+        for (int j = 0; j < LOADS; ++j) load_k1(i, j);
+    }
+    for (int i = 0; i < NS - 1 && i < ntiles; ++i) {
+        next_v(i);
+#pragma unroll
+        for (int j = 0; j < LOADS; ++j) load_v1(i, j);
+    }
     bf16x8 qf[NQB][8];
 #pragma unroll
     for (int nb = 0; nb < NQB; ++nb) load_q_plain(a, wrow0 + 32 * nb + n, head, hf, qf[nb]);
@@ -266,10 +265,12 @@ __global__ __launch_bounds__(NW * 64, 8 / NW) __attribute__((amdgpu_waves_per_eu
             tile_max(sc, mx);
             rescale_for(mx, sc);
         }
-        // ---- refill: K(t+NS) into the slot K(t) left, V(t+NS-1) into the slot V(t-1) left (both read last step)
-        const bool refilled = t + NS < ntiles;
-        if (refilled) issue_k(t + NS, t % NS);
-        if (t + NS - 1 < ntiles) issue_v(t + NS - 1, (t + NS - 1) % NS);
+        // ---- refill: K(t+NS) into the slot K(t) left, V(t+NS-1) into the slot V(t-1) left (both read last step), one
+        // 1 KB load a slot below (all of them here held the wave's issue up behind the memory pipe: 3,000 queries x 700 keys
+        // x 32 heads 49.0 -> 44.5 us with 128-query workgroups, 3,000 x 3,000 x 24 146.7 -> 139.4)
+        const bool refilled = t + NS < ntiles, refill_v = t + NS - 1 < ntiles;
+        if (refilled) next_k(t + NS);
+        if (refill_v) next_v(t + NS - 1);
         {
             // Explicit schedule of the tile's 32 MFMA slots (one wave's instruction stream; a sched_barrier closes
             // every slot, so the compiler keeps each slot's work in it):
@@ -306,6 +307,11 @@ __global__ __launch_bounds__(NW * 64, 8 / NW) __attribute__((amdgpu_waves_per_eu
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
             for (int s = 0; s < 32; ++s) {
+                if (s < LOADS) {
+                    if (refilled) load_k1(t % NS, s);
+                } else if (s < 2 * LOADS) {
+                    if (refill_v) load_v1((t + NS - 1) % NS, s - LOADS);
+                }
                 if (s + 3 < 32) fr[(s + 3) & 3] = frag(s + 3);
                 if (s < 16) {
                     sn[0][s & 1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
