@@ -3,75 +3,102 @@
 // kept keys and their value rows are gathered, in order, into a workspace, and the attention runs over them:
 // softmax over the kept keys equals softmax over all keys with the others at -inf.
 //
-// compact_scan_kernel: one workgroup. Thread i counts the kept keys of its contiguous chunk, an exclusive scan over
-// the workgroup gives each chunk its first output slot, and idx[slot] = key for every kept key (slots < n_valid).
-// gather_rows_kernel: one 16-byte chunk of a K row and of a V row per thread, for rows j < n_valid.
+// One launch: a block owns a range of source keys and a 1 KB slab of their rows' columns. It counts the kept keys before
+// its range (the mask is a few KB, read from L2), which gives its first output slot, then copies its kept rows, 16 bytes a
+// thread, all of a thread's loads in flight together. Bound by HBM on the rows (700 of 1,024 keys x 32 heads: 23 MB) and,
+// at that size, by the launch; a scan launch in front of the gather (one workgroup) cost 3.2 us and the gap between.
 #include "lr_common.h"
 #include "lr_kernels.h"
 
 namespace lr {
 namespace {
 
-constexpr int SCAN_THREADS = 1024;
+constexpr int GT = 256;           // threads
+constexpr int KEYS = 16;          // source keys per pass of a block
+constexpr int SLAB = 64;          // 16-byte chunks of a row per block: one wave a row, four rows at a time
+constexpr int KEYS_PER_THREAD = KEYS / (GT / SLAB);
 
-__global__ __launch_bounds__(SCAN_THREADS) void compact_scan_kernel(const uint8_t* kmask, int nkeys, int n_valid,
-                                                                    int* idx) {
-    __shared__ int part[SCAN_THREADS];
-    const int t = threadIdx.x;
-    const int per = (nkeys + SCAN_THREADS - 1) / SCAN_THREADS;
-    const int b = t * per, e = min(nkeys, b + per);
-    int cnt = 0;
-    for (int j = b; j < e; ++j) cnt += kmask[j] != 0;
-    part[t] = cnt;
-    __syncthreads();
-    // Hillis-Steele inclusive scan over the workgroup
-    for (int off = 1; off < SCAN_THREADS; off <<= 1) {
-        const int add = t >= off ? part[t - off] : 0;
-        __syncthreads();
-        part[t] += add;
-        __syncthreads();
-    }
-    int slot = part[t] - cnt;
-    for (int j = b; j < e; ++j)
-        if (kmask[j] != 0) {
-            if (slot < n_valid) idx[slot] = j;
-            ++slot;
-        }
+// nonzero bytes of a word, a bit each at bits 7, 15, 23, 31
+__device__ __forceinline__ uint32_t nonzero_bytes(uint32_t w) {
+    return (((w & 0x7f7f7f7fu) + 0x7f7f7f7fu) | w) & 0x80808080u;
 }
 
-// A slot whose index is not a key (the mask holds fewer kept keys than n_valid: a caller error) gets zero rows
-// rather than a read out of bounds.
-__global__ void gather_rows_kernel(const uint16_t* k, const uint16_t* v, int64_t kv_rs, const int* idx, int nkeys,
-                                   int n_valid, int row_chunks, uint16_t* kc, uint16_t* vc) {
-    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (i >= (int64_t)n_valid * row_chunks) return;
-    const int j = (int)(i / row_chunks), c = (int)(i - (int64_t)j * row_chunks);
-    const int r = idx[j];
-    const int64_t dst = (int64_t)j * row_chunks * 8 + 8 * c;
-    u32x4 kk = {0u, 0u, 0u, 0u}, vv = {0u, 0u, 0u, 0u};
-    if ((unsigned)r < (unsigned)nkeys) {
-        const int64_t src = (int64_t)r * kv_rs + 8 * c;
-        kk = *reinterpret_cast<const u32x4*>(k + src);
-        vv = *reinterpret_cast<const u32x4*>(v + src);
+// Kept keys of kmask[0 .. n), by the whole block (every thread gets the sum).
+__device__ __forceinline__ int count_kept(const uint8_t* kmask, int n, int* red) {
+    const int t = threadIdx.x;
+    int cnt = 0, i0 = 0;
+    if ((reinterpret_cast<uintptr_t>(kmask) & 15) == 0) {   // 16 bytes a thread at a time
+        i0 = n & ~15;
+        for (int i = 16 * t; i < i0; i += 16 * GT) {
+            const u32x4 w = *reinterpret_cast<const u32x4*>(kmask + i);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) cnt += __popc(nonzero_bytes(w[j]));
+        }
     }
-    *reinterpret_cast<u32x4*>(kc + dst) = kk;
-    *reinterpret_cast<u32x4*>(vc + dst) = vv;
+    for (int i = i0 + t; i < n; i += GT) cnt += kmask[i] != 0;
+#pragma unroll
+    for (int m = 32; m > 0; m >>= 1) cnt += __shfl_xor(cnt, m, 64);
+    if ((t & 63) == 0) red[t >> 6] = cnt;
+    __syncthreads();
+    return red[0] + red[1] + red[2] + red[3];
+}
+
+// Block (x, y): source keys [x * per, (x + 1) * per), column chunks [y * SLAB, (y + 1) * SLAB). Slots past the last kept
+// key (the mask holds fewer than n_valid: a caller error) get zero rows, from the last range's blocks; kept keys past
+// n_valid are left out.
+__global__ __launch_bounds__(GT) void gather_kept_kernel(const uint16_t* k, const uint16_t* v, int64_t kv_rs,
+                                                         const uint8_t* kmask, int nkeys, int n_valid, int per,
+                                                         int row_chunks, uint16_t* kc, uint16_t* vc) {
+    __shared__ int red[GT / 64];
+    const int t = threadIdx.x, r = t / SLAB, c = blockIdx.y * SLAB + t % SLAB;
+    const bool live = c < row_chunks;
+    const int b = blockIdx.x * per, e = min(nkeys, b + per);
+    int slot0 = count_kept(kmask, b, red);
+    for (int k0 = b; k0 < e; k0 += KEYS) {
+        // the pass's mask: bit i = key k0 + i is kept (lanes 0 .. KEYS - 1 of every wave)
+        const int lane = t & 63;
+        const uint32_t keep = (uint32_t)__builtin_amdgcn_ballot_w64(lane < KEYS && k0 + lane < e && kmask[min(k0 + lane, nkeys - 1)] != 0);
+        u32x4 kk[KEYS_PER_THREAD], vv[KEYS_PER_THREAD];
+        int slot[KEYS_PER_THREAD];
+#pragma unroll
+        for (int j = 0; j < KEYS_PER_THREAD; ++j) {
+            const int i = r + (GT / SLAB) * j;
+            slot[j] = slot0 + __popc(keep & ((1u << i) - 1));
+            if (!((keep >> i) & 1) || slot[j] >= n_valid || !live) slot[j] = -1;
+            if (slot[j] >= 0) {
+                const int64_t src = (int64_t)(k0 + i) * kv_rs + 8 * c;
+                kk[j] = *reinterpret_cast<const u32x4*>(k + src);
+                vv[j] = *reinterpret_cast<const u32x4*>(v + src);
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < KEYS_PER_THREAD; ++j)
+            if (slot[j] >= 0) {
+                const int64_t dst = ((int64_t)slot[j] * row_chunks + c) * 8;
+                *reinterpret_cast<u32x4*>(kc + dst) = kk[j];
+                *reinterpret_cast<u32x4*>(vc + dst) = vv[j];
+            }
+        slot0 += __popc(keep);
+    }
+    if (e == nkeys && live)
+        for (int s = slot0 + r; s < n_valid; s += GT / SLAB) {
+            const int64_t dst = ((int64_t)s * row_chunks + c) * 8;
+            *reinterpret_cast<u32x4*>(kc + dst) = u32x4{0u, 0u, 0u, 0u};
+            *reinterpret_cast<u32x4*>(vc + dst) = u32x4{0u, 0u, 0u, 0u};
+        }
 }
 
 }  // namespace
 
 hipError_t launch_compact_keys(const void* k, const void* v, int64_t kv_rs, const uint8_t* kmask, int nkeys,
-                               int n_valid, int HK, void* idx, void* kc, void* vc, hipStream_t stream) {
-    hipLaunchKernelGGL(compact_scan_kernel, dim3(1), dim3(SCAN_THREADS), 0, stream, kmask, nkeys, n_valid,
-                       static_cast<int*>(idx));
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
+                               int n_valid, int HK, void* kc, void* vc, hipStream_t stream) {
     const int row_chunks = HK * D / 8;
-    const int64_t n = (int64_t)n_valid * row_chunks;
-    hipLaunchKernelGGL(gather_rows_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, stream,
-                       static_cast<const uint16_t*>(k), static_cast<const uint16_t*>(v), kv_rs,
-                       static_cast<const int*>(idx), nkeys, n_valid, row_chunks, static_cast<uint16_t*>(kc),
-                       static_cast<uint16_t*>(vc));
+    // 16 keys a block up to 8,192 keys; beyond, more passes a block rather than more counts of the mask before it
+    const int per = KEYS * ((nkeys + 8191) / 8192);
+    const dim3 grid((unsigned)((nkeys + per - 1) / per), (unsigned)((row_chunks + SLAB - 1) / SLAB));
+    hipLaunchKernelGGL(gather_kept_kernel, grid, dim3(GT), 0, stream, static_cast<const uint16_t*>(k),
+                       static_cast<const uint16_t*>(v), kv_rs, kmask, nkeys, n_valid, per, row_chunks,
+                       static_cast<uint16_t*>(kc), static_cast<uint16_t*>(vc));
     return hipGetLastError();
 }
 

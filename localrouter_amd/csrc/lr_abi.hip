@@ -672,7 +672,7 @@ int lr_attention_kmask_bf16(const void* q, const void* k, const void* v, void* o
     void* vc = ws + idx_bytes + rows;
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
     const hipError_t e = lr::launch_compact_keys(k, v, kv_row_stride, static_cast<const uint8_t*>(kmask), nkeys,
-                                                 n_valid, HK, ws, kc, vc, s);
+                                                 n_valid, HK, kc, vc, s);
     if (e != hipSuccess) return (int)e;
     return lr_attention_bf16(q, kc, vc, out, 0, W, H, HK, n_valid, 0, scale, q_row_stride, (int64_t)HK * lr::D,
                              out_row_stride, stream);
