@@ -100,7 +100,12 @@ bool keysplit_fits(int W, int H, int nkeys, int cus, bool split_area) {
 // x 1,577 keys, 32 heads over 8, 32.7 / 40.4 us; 2,048 42.7 / 57.8; 4,096 140 / 187; 4,608 x 24 142 / 178).
 bool keysplit_rows(int W, int H, int nkeys, int causal, int cus, bool split_area) {
     if (nkeys <= 7 * 64 || cus < 1) return false;
-    if ((int64_t)((W + 127) / 128) * H > 1 << 22) return false;   // (a grid's work-items are counted in 32 bits)
+    const int64_t blocks = (int64_t)((W + 127) / 128) * H;
+    if (blocks > 1 << 22) return false;   // (a grid's work-items are counted in 32 bits)
+    // few workgroups over many keys wait for memory, not for each other: two tiles in flight a workgroup are then no
+    // better than the pipelined kernel's ring (64 queries x 32 heads, 4,096 / 32,768 keys 68 / 713 us against 64 / 635;
+    // 128 x 4 heads, 8,192 / 16,384 keys 102 / 243 against 123 / 239; 500 x 16 heads, 32,768 keys 475 against 483)
+    if ((causal || !split_area) && nkeys >= 4096 && (W <= 64 || (nkeys >= 16384 && blocks <= 32))) return false;
     return causal || keysplit_fits(W, H, nkeys, cus, split_area);
 }
 
