@@ -53,31 +53,32 @@ __global__ __launch_bounds__(GT) void gather_kept_kernel(const uint16_t* k, cons
     const int t = threadIdx.x, r = t / SLAB, c = blockIdx.y * SLAB + t % SLAB;
     const bool live = c < row_chunks;
     const int b = blockIdx.x * per, e = min(nkeys, b + per);
-    int slot0 = count_kept(kmask, b, red);
+    const int lane = t & 63;
+    int slot0 = 0;
     for (int k0 = b; k0 < e; k0 += KEYS) {
         // the pass's mask: bit i = key k0 + i is kept (lanes 0 .. KEYS - 1 of every wave)
-        const int lane = t & 63;
-        const uint32_t keep = (uint32_t)__builtin_amdgcn_ballot_w64(lane < KEYS && k0 + lane < e && kmask[min(k0 + lane, nkeys - 1)] != 0);
+        const int km = lane < KEYS && k0 + lane < e ? kmask[k0 + lane] : 0;
+        const uint32_t keep = (uint32_t)__builtin_amdgcn_ballot_w64(km != 0);
         u32x4 kk[KEYS_PER_THREAD], vv[KEYS_PER_THREAD];
-        int slot[KEYS_PER_THREAD];
 #pragma unroll
         for (int j = 0; j < KEYS_PER_THREAD; ++j) {
             const int i = r + (GT / SLAB) * j;
-            slot[j] = slot0 + __popc(keep & ((1u << i) - 1));
-            if (!((keep >> i) & 1) || slot[j] >= n_valid || !live) slot[j] = -1;
-            if (slot[j] >= 0) {
+            if (((keep >> i) & 1) && live) {
                 const int64_t src = (int64_t)(k0 + i) * kv_rs + 8 * c;
                 kk[j] = *reinterpret_cast<const u32x4*>(k + src);
                 vv[j] = *reinterpret_cast<const u32x4*>(v + src);
             }
         }
+        if (k0 == b) slot0 = count_kept(kmask, b, red);   // beside the first rows' loads
 #pragma unroll
-        for (int j = 0; j < KEYS_PER_THREAD; ++j)
-            if (slot[j] >= 0) {
-                const int64_t dst = ((int64_t)slot[j] * row_chunks + c) * 8;
+        for (int j = 0; j < KEYS_PER_THREAD; ++j) {
+            const int i = r + (GT / SLAB) * j, slot = slot0 + __popc(keep & ((1u << i) - 1));
+            if (((keep >> i) & 1) && live && slot < n_valid) {
+                const int64_t dst = ((int64_t)slot * row_chunks + c) * 8;
                 *reinterpret_cast<u32x4*>(kc + dst) = kk[j];
                 *reinterpret_cast<u32x4*>(vc + dst) = vv[j];
             }
+        }
         slot0 += __popc(keep);
     }
     if (e == nkeys && live)
