@@ -36,7 +36,8 @@ __device__ __forceinline__ void kv_tile_block(const KvImageArgs& a, int64_t tile
     const int tid = threadIdx.x, c = tid & 15, g = tid >> 4;
     if (tile_id == 0 && a.cnt)                         // the attention kernel's counters start each call at zero
         for (int x = tid; x < a.ncnt; x += 256) a.cnt[x] = 0;
-    const int hk = (int)(tile_id / a.tiles), t = (int)(tile_id - (int64_t)hk * a.tiles);
+    // (tiles * HK < 2^31, kv_args_ok: a 32-bit division, not the ~100 instructions of a 64-bit one)
+    const int hk = (int)((uint32_t)tile_id / (uint32_t)a.tiles), t = (int)(tile_id - (int64_t)hk * a.tiles);
     const int key0 = t * IMG_TILE_KEYS;
 
     // ---- the loads first: 4 key rows (16 bytes each), the weight, the first key row's table entries (the next row's
@@ -107,8 +108,7 @@ __device__ __forceinline__ void kv_tile_block(const KvImageArgs& a, int64_t tile
         float ss = 0.0f;
 #pragma unroll
         for (int j = 0; j < 8; ++j) ss = fmaf(x[j], x[j], ss);
-#pragma unroll
-        for (int m = 1; m < 16; m <<= 1) ss += __shfl_xor(ss, m, 16);
+        ss = row16_sum(ss);
         const float rr = rsqrtf(ss * (1.0f / D) + a.eps);
         const bool copy = key < a.n_pre;
         float y[8];

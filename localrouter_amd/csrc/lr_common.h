@@ -83,6 +83,35 @@ __device__ __forceinline__ void norm_bf16_exact8(float (&x)[8], double rr, const
     for (int c = 0; c < 8; ++c) x[c] = (float)(bf16)y[c];
 }
 
+// Sum over each row of 16 lanes, in every lane: the partner's partial comes by DPP (a register move inside the row, read
+// straight into the add): quad_perm for lane ^ 1 and lane ^ 2; then, all lanes of a quad holding the same partial, the
+// mirror of 8 lanes brings the other quad's and the mirror of 16 the other half's. The additions are those of the xor
+// butterfly over lane bits 1, 2, 4, 8, bit for bit, without its four LDS round trips (ds_bpermute).
+template <int CTRL>
+__device__ __forceinline__ float dpp_f32(float x) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), CTRL, 0xf, 0xf, true));
+}
+template <int CTRL>
+__device__ __forceinline__ double dpp_f64(double x) {
+    const uint64_t b = (uint64_t)__double_as_longlong(x);
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)b, CTRL, 0xf, 0xf, true);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)(b >> 32), CTRL, 0xf, 0xf, true);
+    return __longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
+}
+constexpr int DPP_XOR1 = 0xb1, DPP_XOR2 = 0x4e, DPP_HALF_MIRROR = 0x141, DPP_MIRROR = 0x140;
+__device__ __forceinline__ float row16_sum(float x) {
+    x += dpp_f32<DPP_XOR1>(x);
+    x += dpp_f32<DPP_XOR2>(x);
+    x += dpp_f32<DPP_HALF_MIRROR>(x);
+    return x + dpp_f32<DPP_MIRROR>(x);
+}
+__device__ __forceinline__ double row16_sum(double x) {
+    x += dpp_f64<DPP_XOR1>(x);
+    x += dpp_f64<DPP_XOR2>(x);
+    x += dpp_f64<DPP_HALF_MIRROR>(x);
+    return x + dpp_f64<DPP_MIRROR>(x);
+}
+
 // Rotation coefficients of pair p at table row `row`: y_a = f00 x_a + f01 x_b, y_b = f10 x_a + f11 x_b.
 struct Rot2 {
     float f00, f01, f10, f11;
