@@ -10,7 +10,7 @@ from __future__ import annotations
 import ctypes
 from pathlib import Path
 
-from . import _lib
+from . import _lib, ops
 
 HEADER = Path(__file__).resolve().parent.parent / "include" / "lr_mmdit.h"
 
@@ -153,14 +153,13 @@ class MMDiTBlock:
             raise _lib.LrError("lr_mmdit_linear_bf16", rc)
 
     def __call__(self, txt, img, t, cos, sin, stream=None):
-        import torch
         n_txt, n_img = txt.shape[0], img.shape[0]
         assert txt.dtype == img.dtype == torch.bfloat16 and txt.is_contiguous() and img.is_contiguous()
         assert t.dtype == torch.float32 and cos.dtype == sin.dtype == torch.float32
         assert cos.shape == (n_txt + n_img, 64) and sin.shape == cos.shape
         ws = self.workspace(n_txt, n_img)
         self.plan(n_txt, n_img)
-        s = torch.cuda.current_stream().cuda_stream if stream is None else stream
+        s = ops._stream() if stream is None else stream
         rc = lib().lr_mmdit_block_bf16(self.ctx, ctypes.byref(self.cw), txt.data_ptr(), img.data_ptr(), n_txt, n_img,
                                        self.hidden, self.mlp, t.data_ptr(), cos.data_ptr(), sin.data_ptr(),
                                        ws.data_ptr(), ws.numel(), s)

@@ -32,8 +32,10 @@ CFG_AUTO, CFG_PIPE_W8, CFG_PIPE_W4, CFG_STREAM_W8 = 0, 1, 2, 9
 SCALE_128 = float(torch.tensor(1.0 / math.sqrt(128.0), dtype=torch.float32))  # f32 1/sqrt(128) = 0x3DB504F3
 
 
+# The current device's current stream as the raw handle. torch.cuda.current_stream().cuda_stream is the same number through
+# a Python Stream object, 2.8 us of a small call's ~17 against 0.2.
 def _stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
 def _ptr(t: torch.Tensor | None):
