@@ -67,6 +67,14 @@ __device__ __forceinline__ void dma4_rows_far(uint64_t addr, uint32_t lds) {
     LR_ASM_M0_END
 }
 
+// n / d for 0 <= n < 2^31, d >= 1, given rcp = floor(2^32 / d) (2^32 - 1 for d = 1): the high product is the quotient or
+// one less. (Four scalar instructions; a division by a value the compiler does not know is ~40, in front of the first
+// load.)
+__device__ __forceinline__ int div_small(int n, int d, uint32_t rcp) {
+    const uint32_t q = (uint32_t)(((uint64_t)(uint32_t)n * rcp) >> 32);
+    return (int)(q + ((uint32_t)n - q * (uint32_t)d >= (uint32_t)d ? 1u : 0u));
+}
+
 template <bool KR>
 __global__ __launch_bounds__(512, 1) __attribute__((amdgpu_waves_per_eu(2, 2))) void attn_keysplit_kernel(AttnArgs a) {
     __shared__ __attribute__((aligned(1024))) uint8_t lds[KS_LDS];
@@ -83,16 +91,16 @@ __global__ __launch_bounds__(512, 1) __attribute__((amdgpu_waves_per_eu(2, 2))) 
     const int nqb = (a.W + KBM - 1) / KBM;
     int head, qblk;
     if (a.causal) {
-        const int h = b % a.H;
-        qblk = nqb - 1 - b / a.H;
+        const int h = b - div_small(b, a.H, a.rcp_h) * a.H;
+        qblk = nqb - 1 - div_small(b, a.H, a.rcp_h);
         head = a.H % 8 == 0 ? (h & 7) * (a.H >> 3) + (h >> 3) : h;
     } else {
         const int per = nwg >> 3, rem8 = nwg & 7, xcd = b & 7, idx = b >> 3;
         const int logical = xcd < rem8 ? xcd * (per + 1) + idx : rem8 * (per + 1) + (xcd - rem8) * per + idx;
-        head = logical / nqb;
+        head = div_small(logical, nqb, a.rcp_nqb);
         qblk = logical - head * nqb;
     }
-    const int hk = head / a.G;
+    const int hk = div_small(head, a.G, a.rcp_g);
     const int row0 = qblk * KBM, wrow0 = row0 + 32 * wv;
     const int T = (a.nkeys + IMG_TILE_KEYS - 1) / IMG_TILE_KEYS;
     const int tb = a.causal ? min(T, (a.p0 + min(row0 + KBM, a.W) - 1) / IMG_TILE_KEYS + 1) : T;
@@ -210,8 +218,8 @@ __global__ __launch_bounds__(512, 1) __attribute__((amdgpu_waves_per_eu(2, 2))) 
         }
     };
 
-    // the two halves' refills of a step, one load every other slot of its first half (all at once would hold the wave's
-    // issue up behind the memory pipe): V(u), then K(u + 1) (past the last tile a repeat of it, never read)
+    // a step's refills, one load every other slot of its first half (all at once would hold the wave's issue up behind
+    // the memory pipe): V(u), then K(u + 1) (past the last tile a repeat of it, never read)
     auto refill = [&](int f, uint64_t vs, uint32_t vd, uint64_t ks, uint32_t kd) __attribute__((always_inline)) {
         if (f % 2 == 0) {
             if (f < 8) load_v1(vs, vd, f / 2);
@@ -226,6 +234,11 @@ __global__ __launch_bounds__(512, 1) __attribute__((amdgpu_waves_per_eu(2, 2))) 
     const float rc = 1.0f / c;
     LR_WAIT_VMCNT(0);
     block_barrier();
+    {
+        const uint64_t vs = v_src(tile_of(0));
+#pragma unroll
+        for (int i = 0; i < 4; ++i) load_v1(vs, vring, i);
+    }
     float mref;
     {
         uint32_t kb0 = ring + lane16, qb0 = qlds + (uint32_t)(8 * wv * IMG_FRAG_BYTES) + lane16;
@@ -253,7 +266,7 @@ __global__ __launch_bounds__(512, 1) __attribute__((amdgpu_waves_per_eu(2, 2))) 
     }
     // ---- step 0: S of half-tile 1 (K(0), fragments 8-15), P of half-tile 0
     {
-        const uint64_t vs = v_src(tile_of(0)), ks = k_src(tile_of(1));
+        const uint64_t ks = k_src(tile_of(1));   // (one tile in all: a repeat of it, never read)
         uint32_t kb = ring + lane16;
         asm volatile("" : "+v"(kb));
         auto rd0 = [&](int f) __attribute__((always_inline)) {
@@ -262,7 +275,7 @@ __global__ __launch_bounds__(512, 1) __attribute__((amdgpu_waves_per_eu(2, 2))) 
 #pragma unroll
         for (int f = 0; f < RA; ++f) rd0(f);
         half_step(s[1], p[1], s[0], p[0], BoolTag<false>{}, [&](int f) __attribute__((always_inline)) {
-            refill(f - RA, vs, vring, ks, ring + IMG_TILE_BYTES);
+            if ((f - RA) % 2 == 0 && f - RA < 8) load_k1(ks, ring + IMG_TILE_BYTES, (f - RA) / 2);
             rd0(f);
         });
         LR_WAIT_VMCNT(0);
@@ -297,37 +310,42 @@ __global__ __launch_bounds__(512, 1) __attribute__((amdgpu_waves_per_eu(2, 2))) 
         LR_WAIT_VMCNT(0);
         block_barrier();
     }
-    // ---- the last half-tile's P and the last value tile's products
-    {
-        const int u = nsteps - 1, j = 2 * (grp + KW * u) + 1;
-        if (j >= jm) mask_half(s[1], j);
-        uint32_t vb0 = vring + (uint32_t)((u & 1) * IMG_TILE_BYTES) + vlane;
-        asm volatile("" : "+v"(vb0));
-        bf16x8 vf[4];
-#pragma unroll
-        for (int x = 0; x < 3; ++x) vf[x] = vfrag_at(vb0 + (uint32_t)vfrag_off(x));
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int x = 0; x < 16; ++x) {
-            if (x + 3 < 16) vf[(x + 3) & 3] = vfrag_at(vb0 + (uint32_t)vfrag_off(x + 3));
-            pv(o[x & 3], vf[x & 3], (x < 8 ? p[0] : p[1])[(x >> 2) & 1]);
-            if (x < 8) {
-                stage_e(s[1], x);
-                stage_c(p[1], x);
-            }
-            __builtin_amdgcn_sched_barrier(0);
-        }
-    }
-
-    // ---- merge: group g writes dims 64 g .. 64 g + 63 of its 32 queries and sends the other 64 to its partner, the
-    // wave of the other group with the same queries. Two code paths (not selects: the accumulators stay where they are).
-    const float l = wave_pair_sum(ls);
-    block_barrier();   // every wave is done with the rings
+    // ---- the last half-tile's P and the last value tile's products, then the merge: group g writes dims 64 g .. 64 g + 63
+    // of its 32 queries and sends the other 64 to its partner, the wave of the other group with the same queries. The
+    // products of the dims to send come first, so that sending them runs beside the last products of the others. (Two
+    // code paths, not selects: the accumulators stay where they are.)
     float* ml = reinterpret_cast<float*>(lds + MG_ML);
     int* flag = reinterpret_cast<int*>(lds + MG_FLAG);
     const int qrow = wrow0 + n;
-    auto merge = [&](auto grp_tag) __attribute__((always_inline)) {
+    auto finish = [&](auto grp_tag) __attribute__((always_inline)) {
         constexpr int G = decltype(grp_tag)::value, SEND = 2 - 2 * G, KEEP = 2 * G;   // 32-dim blocks
+        {
+            const int u = nsteps - 1, j = 2 * (grp + KW * u) + 1;
+            if (j >= jm) mask_half(s[1], j);
+            uint32_t vb0 = vring + (uint32_t)((u & 1) * IMG_TILE_BYTES) + vlane;
+            asm volatile("" : "+v"(vb0));
+            // product x: 16-key step kk(x) of the tile, 32-dim block db(x): the first half-tile's (P of buffer 0), the
+            // dims to send first, then the second half-tile's
+            auto kk = [](int x) __attribute__((always_inline)) { return 2 * (x >> 3) + ((x >> 1) & 1); };
+            auto db = [](int x) __attribute__((always_inline)) { return ((x >> 2) & 1 ? KEEP : SEND) + (x & 1); };
+            auto off = [&](int x) __attribute__((always_inline)) { return (uint32_t)vfrag_off(4 * kk(x) + db(x)); };
+            bf16x8 vf[4];
+#pragma unroll
+            for (int x = 0; x < 3; ++x) vf[x] = vfrag_at(vb0 + off(x));
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int x = 0; x < 16; ++x) {
+                if (x + 3 < 16) vf[(x + 3) & 3] = vfrag_at(vb0 + off(x + 3));
+                pv(o[db(x)], vf[x & 3], (x < 8 ? p[0] : p[1])[(x >> 1) & 1]);
+                if (x < 8) {
+                    stage_e(s[1], x);
+                    stage_c(p[1], x);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+        const float l = wave_pair_sum(ls);
+        block_barrier();   // every wave is done with the rings
         float* mg = reinterpret_cast<float*>(lds + 8192 * wave) + 4 * lane;
         const float* mgp = reinterpret_cast<const float*>(lds + 8192 * (wave ^ QW)) + 4 * lane;
 #pragma unroll
@@ -384,9 +402,9 @@ __global__ __launch_bounds__(512, 1) __attribute__((amdgpu_waves_per_eu(2, 2))) 
     // a row of these 32 overflowed its fixed reference: all of them again with the exact maximum (the queries are still
     // there when they are the output rows: neither wave has written)
     if (grp == 0) {
-        if (merge(IntTag<0>{})) redo_exact<KR>(a, head, hk, row0, tb, wv);
+        if (finish(IntTag<0>{})) redo_exact<KR>(a, head, hk, row0, tb, wv);
     } else {
-        merge(IntTag<1>{});
+        finish(IntTag<1>{});
     }
 }
 
@@ -399,8 +417,13 @@ hipError_t launch_keysplit(const AttnArgs& a, hipStream_t stream, bool key_rows)
         return hipErrorInvalidValue;
     const int64_t blocks = (int64_t)((a.W + KBM - 1) / KBM) * a.H;
     if (blocks > 0x7fffffff) return hipErrorInvalidValue;
-    if (key_rows) hipLaunchKernelGGL(attn_keysplit_kernel<true>, dim3((unsigned)blocks), dim3(512), 0, stream, a);
-    else hipLaunchKernelGGL(attn_keysplit_kernel<false>, dim3((unsigned)blocks), dim3(512), 0, stream, a);
+    auto rcp = [](int64_t d) { return d > 1 ? (uint32_t)(((uint64_t)1 << 32) / (uint64_t)d) : 0xffffffffu; };
+    AttnArgs b = a;
+    b.rcp_nqb = rcp((a.W + KBM - 1) / KBM);
+    b.rcp_h = rcp(a.H);
+    b.rcp_g = rcp(a.G);
+    if (key_rows) hipLaunchKernelGGL(attn_keysplit_kernel<true>, dim3((unsigned)blocks), dim3(512), 0, stream, b);
+    else hipLaunchKernelGGL(attn_keysplit_kernel<false>, dim3((unsigned)blocks), dim3(512), 0, stream, b);
     return hipGetLastError();
 }
 
