@@ -153,6 +153,7 @@ class MMDiTBlock:
             raise _lib.LrError("lr_mmdit_linear_bf16", rc)
 
     def __call__(self, txt, img, t, cos, sin, stream=None):
+        import torch
         n_txt, n_img = txt.shape[0], img.shape[0]
         assert txt.dtype == img.dtype == torch.bfloat16 and txt.is_contiguous() and img.is_contiguous()
         assert t.dtype == torch.float32 and cos.dtype == sin.dtype == torch.float32
