@@ -288,16 +288,27 @@ __device__ __forceinline__ void rope_w_load(const uint16_t* w, int L, float (&wv
 
 __device__ __forceinline__ float bf16_round(float x) { return (float)(bf16)x; }
 
-__device__ __forceinline__ void h3_rms_rope(float (&x)[8], int L, const float (&w)[8], const RopeTab& t, int rot,
-                                            float eps) {
+// The sum of squares of the row a group of 16 lanes holds, in double, in every lane.
+__device__ __forceinline__ double h3_sumsq(const float (&x)[8]) {
     double ss = 0.0;
 #pragma unroll
     for (int c = 0; c < 8; ++c) ss = fma((double)x[c], (double)x[c], ss);
-    ss += xor_lane<1>(ss);
-    ss += xor_lane<2>(ss);
-    ss += xor_lane<4>(ss);
-    ss += xor_lane<8>(ss);
-    norm_bf16_exact8(x, 1.0 / sqrt(ss / 128.0 + (double)eps), w);
+    return row16_sum(ss);
+}
+__device__ __forceinline__ double h3_rrms(double ss, float eps) { return 1.0 / sqrt(ss / 128.0 + (double)eps); }
+// rrms of two rows a group holds one after the other, from their sums of squares: the odd lanes compute the second row's,
+// so that the double square root and division (~45 instructions) run once for both, and a quad broadcast hands them out
+// (the same operations on the same values: the same bits as h3_rrms of each). (Four rows at once kept eight more
+// registers live across the rows: 98, one block a CU fewer, and no gain.)
+__device__ __forceinline__ void h3_rrms2(double ss0, double ss1, float eps, double (&rr)[2]) {
+    const double mine = h3_rrms((threadIdx.x & 1) ? ss1 : ss0, eps);
+    rr[0] = dpp_f64<0xa0>(mine);   // quad_perm [0, 0, 2, 2]
+    rr[1] = dpp_f64<0xf5>(mine);   // quad_perm [1, 1, 3, 3]
+}
+
+__device__ __forceinline__ void h3_rms_rope(float (&x)[8], int L, const float (&w)[8], const RopeTab& t, int rot,
+                                            double rr) {
+    norm_bf16_exact8(x, rr, w);
     const int hc = rot >> 4;
     const bool first = L < hc, second = L >= hc && L < 2 * hc;
     const int partner = first ? L + hc : (second ? L - hc : L);
@@ -378,7 +389,7 @@ __global__ __launch_bounds__(256) void i8_stats_kernel(PrepArgs a) {
             float x[8], wv[8];
             load8(kb + (int64_t)row * a.k_sn + 8 * L, x);
             rope_w_load(a.kw, L, wv);
-            h3_rms_rope(x, L, wv, rope_tab_load(a, row, L), a.rope_rot, a.rope_eps);
+            h3_rms_rope(x, L, wv, rope_tab_load(a, row, L), a.rope_rot, h3_rrms(h3_sumsq(x), a.rope_eps));
 #pragma unroll
             for (int c = 0; c < 8; ++c) rows[grp][8 * L + c] = x[c];
         }
@@ -481,15 +492,24 @@ __device__ void quant_q(const PrepArgs& a, int b, int h, int qb, uint8_t* lds) {
         LR_I8_WAIT_VMCNT(0);   // the table rows (and the lane's own loads)
         __syncthreads();
     }
+    double rr[2];
 #pragma unroll
     for (int i = 0; i < NR; ++i) {
         const int row = qb * QROWS + RPB * i + slot;
         const bool ok = row < a.Sq;
         float x[8];
+        if constexpr (ROPE) {
+            if (i % 2 == 0) {   // this row's and the next one's norm
+                float y[8];
+                unpack8(raw[i], x);
+                unpack8(raw[i + 1], y);
+                h3_rrms2(h3_sumsq(x), h3_sumsq(y), a.rope_eps, rr);
+            }
+        }
         unpack8(raw[i], x);
 #pragma unroll
         for (int c = 0; c < 8; ++c) x[c] = ok ? x[c] : 0.0f;
-        if constexpr (ROPE) h3_rms_rope(x, L, wv, rope_tab_lds(lds, RPB * i + slot, L, a.rope_rot), a.rope_rot, a.rope_eps);
+        if constexpr (ROPE) h3_rms_rope(x, L, wv, rope_tab_lds(lds, RPB * i + slot, L, a.rope_rot), a.rope_rot, rr[i & 1]);
         rotate8<ROT>(x, L);
         float m = 0.0f;
 #pragma unroll
@@ -543,10 +563,13 @@ __device__ void quant_k(const PrepArgs& a, int b, int hk, int kb, uint8_t* lds) 
     for (int ph = 0; ph < NPASS; ph += 2) {
         float x[2][8];
 #pragma unroll
+        for (int j = 0; j < 2; ++j) unpack8(raw[ph + j], x[j]);
+        double rr[2];
+        if constexpr (ROPE) h3_rrms2(h3_sumsq(x[0]), h3_sumsq(x[1]), a.rope_eps, rr);
+#pragma unroll
         for (int j = 0; j < 2; ++j) {
             const int lr = RPB * (ph + j) + prow;   // row within the block
-            unpack8(raw[ph + j], x[j]);
-            if constexpr (ROPE) h3_rms_rope(x[j], L, wv, rope_tab_lds(lds, lr, L, a.rope_rot), a.rope_rot, a.rope_eps);
+            if constexpr (ROPE) h3_rms_rope(x[j], L, wv, rope_tab_lds(lds, lr, L, a.rope_rot), a.rope_rot, rr[j]);
 #pragma unroll
             for (int c = 0; c < 8; ++c) x[j][c] = x[j][c] - av[c];
             rotate8<ROT>(x[j], L);
