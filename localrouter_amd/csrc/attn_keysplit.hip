@@ -259,7 +259,8 @@ __global__ __launch_bounds__(512, 1) __attribute__((amdgpu_waves_per_eu(2, 2))) 
         for (int q = 1; q < 16; ++q) mx = fmaxf(mx, s[0][q]);
         mx = wave_pair_max(mx);
         mref = mx > -INFINITY ? ceilf(mx * c) : 0.0f;
-        const float mc = mref * rc;   // (its rounding shifts every exponent of the row alike)
+        float mc = mref * rc;   // (its rounding shifts every exponent of the row alike, so it is rounded once: opaque, or
+        asm volatile("" : "+v"(mc));   // the subtraction below could take the product unrounded)
         negm = f32x16{} - mc;
         s[0] -= mc;
         asm volatile(LR_NOP48 : "+v"(negm));
@@ -367,7 +368,7 @@ __global__ __launch_bounds__(512, 1) __attribute__((amdgpu_waves_per_eu(2, 2))) 
         const float M = fmaxf(l0 > 0.0f ? m0 : -INFINITY, l1 > 0.0f ? m1 : -INFINITY);
         float w0 = l0 > 0.0f ? __builtin_amdgcn_exp2f(m0 - M) : 0.0f;
         float w1 = l1 > 0.0f ? __builtin_amdgcn_exp2f(m1 - M) : 0.0f;
-        const float inv = 1.0f / (w0 * l0 + w1 * l1);
+        const float inv = 1.0f / fmaf(w1, l1, w0 * l0);   // (spelled out: every instantiation rounds alike)
         w0 *= inv;
         w1 *= inv;
         const float wm = G == 0 ? w0 : w1, wp = G == 0 ? w1 : w0;
