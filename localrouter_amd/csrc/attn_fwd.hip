@@ -174,6 +174,29 @@ __global__ __launch_bounds__(NW * 64, 8 / NW) __attribute__((amdgpu_waves_per_eu
     // ---- K(0 .. NS-1) and V(0 .. NS-2) resident; S(0)
     LR_WAIT_VMCNT(0);
     block_barrier();
+    // A wave none of whose query rows exist only moves its share of the tiles (the refills and barriers of the steps
+    // below): its products would cost issue slots and power. 218 queries in a 256-query block have one, a decode step three
+    // of four.
+    if (wrow0 >= a.W) {
+        block_barrier();
+        for (int t = 0; t < ntiles; ++t) {
+            const bool refilled = t + NS < ntiles;
+            if (refilled) {
+                next_k(t + NS);
+#pragma unroll
+                for (int j = 0; j < LOADS; ++j) load_k1(t % NS, j);
+            }
+            if (t + NS - 1 < ntiles) {
+                next_v(t + NS - 1);
+#pragma unroll
+                for (int j = 0; j < LOADS; ++j) load_v1((t + NS - 1) % NS, j);
+            }
+            if (NS == 2 || !refilled) LR_WAIT_VMCNT(0);
+            else LR_WAIT_VMCNT((NS - 2) * 2 * LOADS);
+            block_barrier();
+        }
+        return;
+    }
     f32x16 sA[NQB][MB], sB[NQB][MB];
 #pragma unroll
     for (int nb = 0; nb < NQB; ++nb)
@@ -403,24 +426,38 @@ __global__ __launch_bounds__(NW * 64, 8 / NW) __attribute__((amdgpu_waves_per_eu
 }
 
 // One wave per (head, query row): O = sum_s 2^(m_s - M) O_s / sum_s 2^(m_s - M) l_s, M = max_s m_s, two dims a lane.
-__global__ void attn_split_combine_kernel(AttnArgs a) {
+// Lane s holds range s's reference, row sum and weight (at most 64 ranges), so that the partial rows are read with no
+// load depending on another, eight in flight (a loop over the ranges, each with its reference read first, took 13.1 us for
+// 218 queries x 16 heads x 16 ranges, 28.6 MB).
+__global__ __launch_bounds__(256) void attn_split_combine_kernel(AttnArgs a) {
     const int64_t r = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
     const int lane = threadIdx.x & 63;
     if (r >= (int64_t)a.H * a.W) return;
     const int head = (int)(r / a.W), qrow = (int)(r - (int64_t)head * a.W);
     const int ns = a.nsplit;
     const float* ml = a.part_ml + r * ns * 2;
-    float M = -INFINITY;
-    for (int s = 0; s < ns; ++s) M = fmaxf(M, ml[2 * s]);
-    float L = 0.0f, o0 = 0.0f, o1 = 0.0f;
-    for (int s = 0; s < ns; ++s) {
-        const float m = ml[2 * s];
-        if (m == -INFINITY) continue;
-        const float w = __builtin_amdgcn_exp2f(m - M);
-        L = fmaf(w, ml[2 * s + 1], L);
-        const float* po = a.part_o + (r * ns + s) * D + 2 * lane;
-        o0 = fmaf(w, po[0], o0);
-        o1 = fmaf(w, po[1], o1);
+    const float* po = a.part_o + r * ns * D + 2 * lane;
+    const bool live = lane < ns;
+    const float m = live ? ml[2 * lane] : -INFINITY, l = live ? ml[2 * lane + 1] : 0.0f;
+    float M = m;
+#pragma unroll
+    for (int x = 32; x > 0; x >>= 1) M = fmaxf(M, __shfl_xor(M, x, 64));
+    const float w = m > -INFINITY ? __builtin_amdgcn_exp2f(m - M) : 0.0f;   // (an empty range: no weight)
+    float L = w * l;
+#pragma unroll
+    for (int x = 32; x > 0; x >>= 1) L += __shfl_xor(L, x, 64);
+    float o0 = 0.0f, o1 = 0.0f;
+    for (int s0 = 0; s0 < ns; s0 += 8) {
+        float2 v[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) v[j] = *reinterpret_cast<const float2*>(po + (int64_t)min(s0 + j, ns - 1) * D);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const float ws = s0 + j < ns ? __shfl(w, s0 + j, 64) : 0.0f;
+            // (an empty range's row is zeros, or in a range of only masked work whatever it holds: weight 0 leaves it out)
+            o0 = ws > 0.0f ? fmaf(ws, v[j].x, o0) : o0;
+            o1 = ws > 0.0f ? fmaf(ws, v[j].y, o1) : o1;
+        }
     }
     const float inv = 1.0f / L;
     *reinterpret_cast<uint32_t*>(a.out + (int64_t)qrow * a.o_rs + head * D + 2 * lane) = pack_bf16x2(o0 * inv, o1 * inv);

@@ -1164,16 +1164,26 @@ __global__ __launch_bounds__(256) void i8_split_combine_kernel(AttnArgs a) {
     const int q = qblk * 256 + ql;
     if (q >= a.Sq) return;
     const float* ml = a.part + (size_t)a.p.part_n * 256 * HD;
-    float M = -INFINITY;
-    for (int r = 0; r < a.P; ++r) M = fmaxf(M, ml[((size_t)(i * a.P + r) * 256 + ql) * 2]);
+    // every piece's reference, row sum and dims in flight together (pieces past P: piece 0 again, weight 0)
+    float2 mlr[SPLIT_MAX], ov[SPLIT_MAX];
+#pragma unroll
+    for (int r = 0; r < SPLIT_MAX; ++r) {
+        const size_t pr = (size_t)(i * a.P + (r < a.P ? r : 0)) * 256 + ql;
+        mlr[r] = *reinterpret_cast<const float2*>(ml + 2 * pr);
+        ov[r] = *reinterpret_cast<const float2*>(a.part + pr * HD + 2 * lane);
+    }
+    float M = mlr[0].x;
+#pragma unroll
+    for (int r = 1; r < SPLIT_MAX; ++r) M = fmaxf(M, mlr[r].x);
     float L = 0.0f, o0 = 0.0f, o1 = 0.0f;
-    for (int r = 0; r < a.P; ++r) {
-        const size_t pr = (size_t)(i * a.P + r) * 256 + ql;
-        const float w = __builtin_amdgcn_exp2f(ml[2 * pr] - M);
-        L = fmaf(w, ml[2 * pr + 1], L);
-        const float2 ov = *reinterpret_cast<const float2*>(a.part + pr * HD + 2 * lane);
-        o0 = fmaf(w, ov.x, o0);
-        o1 = fmaf(w, ov.y, o1);
+#pragma unroll
+    for (int r = 0; r < SPLIT_MAX; ++r) {
+        if (r < a.P) {
+            const float w = __builtin_amdgcn_exp2f(mlr[r].x - M);
+            L = fmaf(w, mlr[r].y, L);
+            o0 = fmaf(w, ov[r].x, o0);
+            o1 = fmaf(w, ov[r].y, o1);
+        }
     }
     const float inv = 1.0f / L;
     *reinterpret_cast<uint32_t*>(a.out + b * a.o_sb + head * a.o_sh + (int64_t)q * a.o_sn + 2 * lane) =
