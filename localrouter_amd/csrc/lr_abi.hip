@@ -138,8 +138,17 @@ int attention_impl(const void* q, const void* k, const void* v, void* out, int p
     a.W = W; a.H = H; a.HK = HK; a.G = H / HK; a.nkeys = nkeys; a.p0 = p0; a.causal = causal;
     a.c = scale * 1.4426950408889634f;
     const int ns = split_count(W, H, nkeys, causal);
+    const int cus = config == LR_ATTN_CFG_AUTO || config == LR_ATTN_CFG_STREAM_W8 ? device_cus() : 0;
+    const bool ws_split_area = workspace && ws_bytes >= (size_t)LR_JOINT_SPLIT_BYTES && aligned(workspace, 256);
+    // (the key-split kernel takes 32-bit per-lane row offsets, as the streaming kernel does: wider strides go on)
+    const bool keysplit = config == LR_ATTN_CFG_AUTO && keysplit_rows(W, H, nkeys, causal, cus, ws_split_area) &&
+                          k_rs <= lr::STREAM_MAX_V_RS && v_rs <= lr::STREAM_MAX_V_RS;
+    // up to 24 key tiles the key-split kernel is as fast as the split over workgroups and its merge launch (500 queries x
+    // 1,100 keys x 16 heads 20.7 / 30.0 us, 150 x 1,000 x 32 19.1 / 22.9, 218 x 1,500 x 16 24.4 / 24.6; 2,500 keys 35.0 /
+    // 27.3)
     const bool split = workspace && ns > 1 && (config == LR_ATTN_CFG_AUTO || config == LR_ATTN_CFG_PIPE_W8) &&
-                       k_hs == lr::D && v_hs == lr::D && ws_bytes >= split_bytes(W, H, ns) && aligned(workspace, 256);
+                       !(keysplit && nkeys <= 24 * 64) && k_hs == lr::D && v_hs == lr::D &&
+                       ws_bytes >= split_bytes(W, H, ns) && aligned(workspace, 256);
     if (split) {
         a.nsplit = ns;
         a.part_o = static_cast<float*>(workspace);
@@ -149,12 +158,7 @@ int attention_impl(const void* q, const void* k, const void* v, void* out, int p
         if (e != hipSuccess) return (int)e;
         return (int)lr::launch_split_combine(a, stream);
     }
-    const bool ws_split_area = workspace && ws_bytes >= (size_t)LR_JOINT_SPLIT_BYTES && aligned(workspace, 256);
-    // (the key-split kernel takes 32-bit per-lane row offsets, as the streaming kernel does: wider strides go on)
-    const int cus = config == LR_ATTN_CFG_AUTO || config == LR_ATTN_CFG_STREAM_W8 ? device_cus() : 0;
-    if (config == LR_ATTN_CFG_AUTO && keysplit_rows(W, H, nkeys, causal, cus, ws_split_area) &&
-        k_rs <= lr::STREAM_MAX_V_RS && v_rs <= lr::STREAM_MAX_V_RS)
-        return (int)lr::launch_keysplit(a, stream, true);
+    if (keysplit) return (int)lr::launch_keysplit(a, stream, true);
     if (config == LR_ATTN_CFG_AUTO && stream_rows(W, H, nkeys, causal, ws_split_area, cus)) {
         config = LR_ATTN_CFG_STREAM_W8;
     } else if (config == LR_ATTN_CFG_AUTO) {
