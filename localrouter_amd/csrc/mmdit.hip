@@ -209,41 +209,80 @@ __global__ void ksum_residual_kernel(uint16_t* x, const float* part, int rows, i
     store8(xr, xv);
 }
 
-// y[n] = sum_k x[k] w[n, k] for one input row (the time and modulation vectors): HBM-bound on w, one wave per
-// output, 16-byte loads along the weight row, a butterfly sum. K a multiple of 8. SILU: y = SiLU of the bf16 result,
-// the arithmetic of silu_kernel (the time MLP's two activations without launches of their own). SIN: x is the time
-// sinusoid of *t (K = 256), each element computed where it is used, as time_sinusoid_kernel computes it.
+// y[n] = sum_k x[k] w[n, k] for one input row (the time and modulation vectors): HBM-bound on w, one wave per output,
+// 16-byte loads along the weight row, four of them in flight, a butterfly sum. K a multiple of 8. SILU: y = SiLU of the
+// bf16 result, the arithmetic of silu_kernel (the time MLP's two activations without launches of their own). Outputs from
+// n0 on come from w2 into y2 (the two streams' modulations in one launch).
 constexpr int GEMV_WAVES = 4;
-template <bool SILU, bool SIN = false>
-__global__ __launch_bounds__(64 * GEMV_WAVES) void gemv_kernel(const uint16_t* x, const uint16_t* w, uint16_t* y, int N,
-                                                               int K, const float* t = nullptr) {
-    const int n = blockIdx.x * GEMV_WAVES + (threadIdx.x >> 6), lane = threadIdx.x & 63;
-    if (n >= N) return;
-    const uint16_t* row = w + (int64_t)n * K;
-    float tr = 0.0f;
-    if constexpr (SIN) tr = time_scaled(t);
+__device__ __forceinline__ float gemv_row(const uint16_t* x, const uint16_t* row, int K, int lane) {
     float acc = 0.0f;
-    for (int c = lane; c < K / 8; c += 64) {
-        const Chunk8 a = load8(row + 8 * c);
-        Chunk8 b;
-        if constexpr (SIN) {
+    const int nc = K / 8;
+    int c = lane;
+    for (; c + 192 < nc; c += 256) {
+        Chunk8 a[4], b[4];
 #pragma unroll
-            for (int e = 0; e < 8; ++e) b.v[e] = bf(sinusoid_at(tr, 8 * c + e));
-        } else {
-            b = load8(x + 8 * c);
-        }
+        for (int j = 0; j < 4; ++j) a[j] = load8(row + 8 * (c + 64 * j));
+#pragma unroll
+        for (int j = 0; j < 4; ++j) b[j] = load8(x + 8 * (c + 64 * j));
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+            for (int e = 0; e < 8; ++e) acc = fmaf(a[j].v[e], b[j].v[e], acc);
+    }
+    for (; c < nc; c += 64) {
+        const Chunk8 a = load8(row + 8 * c), b = load8(x + 8 * c);
 #pragma unroll
         for (int e = 0; e < 8; ++e) acc = fmaf(a.v[e], b.v[e], acc);
     }
+    return acc;
+}
+template <bool SILU>
+__device__ __forceinline__ uint16_t gemv_out(float acc) {
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) acc += __shfl_xor(acc, o, 64);
-    if (lane == 0) {
-        if constexpr (SILU) {
-            const float v = bf(tobf(acc));
-            y[n] = tobf(v / (1.0f + expf(-v)));
-        } else {
-            y[n] = tobf(acc);
-        }
+    if constexpr (SILU) {
+        const float v = bf(tobf(acc));
+        return tobf(v / (1.0f + expf(-v)));
+    } else {
+        return tobf(acc);
+    }
+}
+template <bool SILU>
+__global__ __launch_bounds__(64 * GEMV_WAVES) void gemv_kernel(const uint16_t* x, const uint16_t* w, uint16_t* y, int N,
+                                                               int K, const uint16_t* w2, uint16_t* y2, int n0) {
+    int n = blockIdx.x * GEMV_WAVES + (threadIdx.x >> 6);
+    const int lane = threadIdx.x & 63;
+    if (n >= N) return;
+    if (n >= n0) {
+        n -= n0;
+        w = w2;
+        y = y2;
+    }
+    const uint16_t v = gemv_out<SILU>(gemv_row(x, w + (int64_t)n * K, K, lane));
+    if (lane == 0) y[n] = v;
+}
+// The first of the time MLP's: x is the time sinusoid of *t (K = 256), computed where it is used as time_sinusoid_kernel
+// computes it, each lane the four elements it multiplies, once for the SIN_OUTS outputs of its wave (a wave per output and
+// eight elements on half the lanes spent 7 us on sines and cosines).
+constexpr int SIN_OUTS = 4;
+__global__ __launch_bounds__(64 * GEMV_WAVES) void gemv_sinusoid_kernel(const uint16_t* w, uint16_t* y, int N, const float* t) {
+    const int n = (blockIdx.x * GEMV_WAVES + (threadIdx.x >> 6)) * SIN_OUTS, lane = threadIdx.x & 63;
+    if (n >= N) return;
+    u32x2 r[SIN_OUTS];
+#pragma unroll
+    for (int j = 0; j < SIN_OUTS; ++j) r[j] = *reinterpret_cast<const u32x2*>(w + (int64_t)min(n + j, N - 1) * 256 + 4 * lane);
+    const float tr = time_scaled(t);
+    float b[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) b[e] = bf(sinusoid_at(tr, 4 * lane + e));
+#pragma unroll
+    for (int j = 0; j < SIN_OUTS; ++j) {
+        float acc = lo_bf16(r[j][0]) * b[0];
+        acc = fmaf(hi_bf16(r[j][0]), b[1], acc);
+        acc = fmaf(lo_bf16(r[j][1]), b[2], acc);
+        acc = fmaf(hi_bf16(r[j][1]), b[3], acc);
+        const uint16_t v = gemv_out<true>(acc);
+        if (lane == 0 && n + j < N) y[n + j] = v;
     }
 }
 
@@ -417,7 +456,7 @@ int gemm(Ctx& c, const void* X, int64_t ldx, const void* W, void* Y, int64_t ldy
     if (is_vector(M, K, X, W)) {   // a vector: HBM-bound
         hipLaunchKernelGGL(gemv_kernel<false>, dim3((unsigned)((N + GEMV_WAVES - 1) / GEMV_WAVES)), dim3(64 * GEMV_WAVES), 0,
                            s, static_cast<const uint16_t*>(X), static_cast<const uint16_t*>(W),
-                           static_cast<uint16_t*>(Y), (int)N, (int)K);
+                           static_cast<uint16_t*>(Y), (int)N, (int)K, nullptr, nullptr, (int)N);
         return (int)hipGetLastError();
     }
     GemmPlan* p = nullptr;
@@ -688,7 +727,8 @@ int lr_mmdit_block_bf16(void* ctx, const lr_mmdit_weights* w, void* txt, void* i
     auto linear_silu = [&](const uint16_t* x_, const void* w_, uint16_t* pre, uint16_t* y_, int64_t N, int64_t K) -> int {
         if (is_vector(1, K, x_, w_)) {
             hipLaunchKernelGGL(gemv_kernel<true>, dim3((unsigned)((N + GEMV_WAVES - 1) / GEMV_WAVES)),
-                               dim3(64 * GEMV_WAVES), 0, s, x_, static_cast<const uint16_t*>(w_), y_, (int)N, (int)K);
+                               dim3(64 * GEMV_WAVES), 0, s, x_, static_cast<const uint16_t*>(w_), y_, (int)N, (int)K,
+                               nullptr, nullptr, (int)N);
             return (int)hipGetLastError();
         }
         int r = gemm(c, x_, K, w_, pre, N, 1, N, K, gws, s);
@@ -698,8 +738,8 @@ int lr_mmdit_block_bf16(void* ctx, const lr_mmdit_weights* w, void* txt, void* i
         return (int)hipGetLastError();
     };
     if (is_vector(1, 256, emb, w->t1)) {   // sinusoid -> linear -> SiLU in one launch
-        hipLaunchKernelGGL((gemv_kernel<true, true>), dim3((unsigned)((D + GEMV_WAVES - 1) / GEMV_WAVES)),
-                           dim3(64 * GEMV_WAVES), 0, s, nullptr, static_cast<const uint16_t*>(w->t1), h1, (int)D, 256, t);
+        hipLaunchKernelGGL(gemv_sinusoid_kernel, dim3((unsigned)((D + GEMV_WAVES * SIN_OUTS - 1) / (GEMV_WAVES * SIN_OUTS))),
+                           dim3(64 * GEMV_WAVES), 0, s, static_cast<const uint16_t*>(w->t1), h1, (int)D, t);
         LR_LAUNCHED();
     } else {
         hipLaunchKernelGGL(time_sinusoid_kernel, dim3(1), dim3(256), 0, s, t, emb);
@@ -707,8 +747,11 @@ int lr_mmdit_block_bf16(void* ctx, const lr_mmdit_weights* w, void* txt, void* i
         LR_TRY(linear_silu(emb, w->t1, h1, h1, D, 256));
     }
     LR_TRY(linear_silu(h1, w->t2, temb, ts, D, D));
-    LR_TRY(gemm(c, ts, D, w->txt.mod, mod_txt, 6 * D, 1, 6 * D, D, gws, s));
-    LR_TRY(gemm(c, ts, D, w->img.mod, mod_img, 6 * D, 1, 6 * D, D, gws, s));
+    // the two streams' modulations in one launch (D is a multiple of 128 and the pointers are 16-byte aligned: vectors)
+    hipLaunchKernelGGL(gemv_kernel<false>, dim3((unsigned)((12 * D + GEMV_WAVES - 1) / GEMV_WAVES)), dim3(64 * GEMV_WAVES), 0,
+                       s, ts, static_cast<const uint16_t*>(w->txt.mod), mod_txt, (int)(12 * D), (int)D,
+                       static_cast<const uint16_t*>(w->img.mod), mod_img, (int)(6 * D));
+    LR_LAUNCHED();
 
     // attention half: LN + modulation (both streams, one launch), QKV per stream into the joint rows
     hipLaunchKernelGGL(ln_modulate_kernel<false>, dim3((unsigned)S), dim3(LN_THREADS), 0, s, xt, xi, n_txt, (int)D,
