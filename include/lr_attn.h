@@ -114,9 +114,10 @@ int lr_attention_bf16_ex(const void* q, const void* k, const void* v, void* out,
                          int config, lr_stream_t stream);
 
 /*
- * lr_attention_bf16 with device scratch. A non-causal call with at most 32 blocks of 256 queries x heads and at least
- * 961 keys (16 tiles of 64; e.g. 218 queries over 50,220 keys) is split over the keys into ranges that fill the GPU,
- * each range's partial result written to the workspace, then merged (flash-decoding). Other non-causal calls of at least
+ * lr_attention_bf16 with device scratch. A non-causal call with at most 32 blocks of 256 queries x heads and more than
+ * 1,536 keys (24 tiles of 64; e.g. 218 queries over 50,220 keys), or at least 961 where the key-split kernel does not
+ * cover the call, is split over the keys into ranges that fill the GPU, each range's partial result written to the
+ * workspace, then merged (flash-decoding). Other non-causal calls of at least
  * 4,096 keys (but for those of few query blocks whose keys the key-split kernel covers sooner) run
  * LR_ATTN_CFG_STREAM_W8 over the key rows, whose last partial round of query blocks is cut over all workgroups
  * along the keys, the pieces' partials and arrival counters in the workspace (LR_JOINT_SPLIT_BYTES; the call clears

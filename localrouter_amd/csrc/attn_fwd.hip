@@ -18,9 +18,9 @@
 //  * The kernel (attn_fwd_pipe_kernel) keeps K and V tiles row-major in an LDS ring filled by direct global->LDS
 //    loads and reads V transposed (ds_read_b64_tr_b16); the QK^T MFMAs of the next tile run interleaved with the
 //    softmax VALU work of the current one. 8-wave blocks (256 queries, two waves per SIMD) or 4-wave blocks (two per
-//    CU). The fused joint attention runs the streaming kernel of attn_stream.hip instead.
+//    CU). The fused joint attention runs the streaming kernel of attn_stream.hip or the key-split kernel of
+//    attn_keysplit.hip instead; calls over rows take either of those too where lr_abi.hip's rules say so.
 //  * Workgroups are remapped so that each XCD works on whole heads (its own L2 holds that head's K/V).
-//  * FUSEQ: the query block's per-head RMSNorm and RoPE are applied in registers before the first MFMA.
 #include "lr_common.h"
 #include "lr_kernels.h"
 

@@ -62,7 +62,8 @@ enum AttnConfig : int {
 
 // Plain attention over value rows (AUTO = PIPE_W8; a.nsplit > 1 splits every query block over the keys).
 hipError_t launch_attention(const AttnArgs& a, int config, hipStream_t stream);
-// keys.hip: gather the kept keys (kmask[j] != 0, in order) and their value rows into kc / vc [n_valid][HK * 128]
+// keys.hip: gather the kept keys (kmask[j] != 0, in order) and their value rows into kc / vc [n_valid][HK * 128], one
+// launch
 hipError_t launch_compact_keys(const void* k, const void* v, int64_t kv_rs, const uint8_t* kmask, int nkeys,
                                int n_valid, int HK, void* kc, void* vc, hipStream_t stream);
 // Merge the key-split partials of a launch with a.nsplit > 1 into out (bf16 rows).
