@@ -67,45 +67,31 @@ __device__ __forceinline__ uint32_t lds_addr(const void* p) {
 }
 
 // ------------------------------------------------------------------------------------------------ prep helpers
-// Exchange with lane ^ M. M < 16: inside each row of 16 lanes by DPP (a register move across lanes, no LDS round
-// trip): quad_perm [1,0,3,2] / [2,3,0,1] for M = 1 / 2, row_ror:8 for M = 8 (a rotation by 8 inside a 16-lane row is
-// xor 8); for M = 4 the lanes with bit 2 clear take row_shl:4 (lane i + 4), the others row_shr:4 (lane i - 4). M = 16:
-// inside each 32-lane half (ds_swizzle, and 0x1f, xor 16).
+// Exchange across lanes by DPP (a register move, no LDS round trip): quad_perm [1,0,3,2] / [2,3,0,1] for lane ^ 1 / ^ 2,
+// row_half_mirror for lane ^ 7, row_ror:8 for lane ^ 8 (a rotation by 8 inside a 16-lane row), and, inside each 32-lane
+// half, ds_swizzle (and 0x1f, xor 16) for lane ^ 16. No single move is lane ^ 4.
 template <int CTRL>
 __device__ __forceinline__ int dpp_mov(int x) {
     return __builtin_amdgcn_update_dpp(0, x, CTRL, 0xf, 0xf, true);
 }
-// the DPP control of the single-move exchanges (M = 1, 2, 8)
-template <int M>
-constexpr int xor_dpp_ctrl() { return M == 1 ? 0xb1 : M == 2 ? 0x4e : 0x128; }
-template <int M>
-__device__ __forceinline__ int xor_lane_i(int x) {
-    if constexpr (M == 1 || M == 2 || M == 8) {
-        return dpp_mov<xor_dpp_ctrl<M>()>(x);
-    } else if constexpr (M == 4) {
-        const int up = dpp_mov<0x104>(x), dn = dpp_mov<0x114>(x);
-        return (threadIdx.x & 4) ? dn : up;
-    } else {
-        return __builtin_amdgcn_ds_swizzle(x, 0x1f | (M << 10));
-    }
-}
 template <int M>
 __device__ __forceinline__ float xor_lane(float x) {
-    return __int_as_float(xor_lane_i<M>(__float_as_int(x)));
+    const int b = __float_as_int(x);
+    if constexpr (M == 16) return __int_as_float(__builtin_amdgcn_ds_swizzle(b, 0x1f | (M << 10)));
+    else return __int_as_float(dpp_mov<M == 1 ? 0xb1 : M == 2 ? 0x4e : M == 7 ? 0x141 : 0x128>(b));
 }
-template <int M>
-__device__ __forceinline__ double xor_lane(double x) {
-    const uint64_t b = (uint64_t)__double_as_longlong(x);
-    const uint32_t lo = (uint32_t)xor_lane_i<M>((int)(uint32_t)b), hi = (uint32_t)xor_lane_i<M>((int)(uint32_t)(b >> 32));
-    return __longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
-}
+
+// The 8-channel group a lane of a row's 8 or 16 holds: lanes with bit 2 set hold theirs mirrored inside the quad, so that
+// the group 4 away is on lane ^ 7 (one DPP move, where lane ^ 4 is two and a select). Its own inverse; groups 1, 2 and 8
+// away stay on lane ^ 1, ^ 2 and ^ 8.
+__device__ __forceinline__ int group_lane(int l) { return (l & 4) ? l ^ 3 : l; }
 
 // max over each group of LPR lanes (one row of 8 * LPR channels, 8 per lane)
 template <int LPR>
 __device__ __forceinline__ float max_row(float x) {
     x = fmaxf(x, xor_lane<1>(x));
     x = fmaxf(x, xor_lane<2>(x));
-    x = fmaxf(x, xor_lane<4>(x));
+    x = fmaxf(x, xor_lane<7>(x));   // (the maximum of the other quad, on each of its lanes)
     if (LPR == 16) x = fmaxf(x, xor_lane<8>(x));
     return x;
 }
@@ -118,14 +104,13 @@ __device__ __forceinline__ float max64(float x) {
     return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
 }
 
-// Round to nearest even, saturate to [-128, 127]; NaN -> 0 (float_utils.cuh:40-51). v_cvt_i32_f32 itself turns NaN
-// into 0 and saturates out-of-range values (infinities included) to the int32 range, so after the rounding one
-// integer clamp remains (written as asm: the conversion of NaN or of an out-of-range value is undefined in C++).
-__device__ __forceinline__ int rn_sat(float x) {
-    int i;
-    asm("v_cvt_i32_f32 %0, %1" : "=v"(i) : "v"(rintf(x)));
-    return min(max(i, -128), 127);
-}
+// The low byte of the result is x rounded to the nearest even integer, in two's complement, for |x| < 2^21; NaN -> 0
+// (float_utils.cuh:40-51 rounds, turns NaN into 0 and saturates to [-128, 127]). Adding 1.5 * 2^23 rounds x to an integer
+// in the sum's low mantissa bits. Nothing saturates here: x is a value times 1 / (its group's largest magnitude / 127 +
+// something positive), so |x| is at most 127 (1 + 2^-22), or NaN where the group holds an infinity (times 0). A NaN's low
+// 16 bits are zero: it comes from a bf16 input or from the arithmetic, whose own is 0x7fc00000. (One add in place of a
+// rounding, a conversion and a clamp.)
+__device__ __forceinline__ int rn_byte(float x) { return __float_as_int(x + 12582912.0f); }
 
 // The low bytes of four ints as one little-endian word (v_perm_b32: byte selector 0x0c is zero)
 __device__ __forceinline__ uint32_t pack_lo_bytes(int b0, int b1, int b2, int b3) {
@@ -137,29 +122,44 @@ __device__ __forceinline__ uint32_t pack_lo_bytes(int b0, int b1, int b2, int b3
 // The reference rotates a 128-channel row held as 4 channels per lane of 32 lanes (quant_qk_int8.cu:75-155):
 // [sign flip], H4 on the lane's 4 channels, [five butterflies over lane bits 1, 2, 4, 8, 16, then * 1/sqrt(128)];
 // a 64-channel row (convrot64) as 4 channels per lane of 16 lanes: H4, four butterflies over lane bits 1 .. 8, * 1/4.
-// Here a lane L of a group of 16 (8 at head dim 64) holds 8 channels, those of the reference's lanes r = 2L and
+// Here lane group_lane(L) of a row's 16 (8 at head dim 64) holds 8 channels, those of the reference's lanes r = 2L and
 // 2L + 1: the sign flip and the H4 act on each 4-channel half, the butterfly over lane bit 1 pairs the two halves in
 // registers, and those over lane bits 2 .. 16 (2 .. 8) are butterflies over L's bits 1 .. 8 (1 .. 4). Every value
 // sees the same operations in the same order as in the reference, so the results are the same bits.
-// A butterfly gives the lane with bit M clear x + o and the other o - x (o the partner's value). For M = 1, 2, 8 the
-// partner is one DPP move away, so it is o + (+-x): this lane's value with its sign flipped where bit M is set (exactly
-// o - x in IEEE arithmetic), and the partner's value read straight into the add (v_add_f32_dpp): two instructions a
-// value. For M = 4 the two directions are separate shifts: x + (lane i + 4) and (lane i - 4) - x, each with the shifted
-// operand read into the add / subtract, then one select.
-template <int M>
-__device__ __forceinline__ void butterfly8(float (&x)[8], int L) {
-#pragma clang fp contract(off)
-    const uint32_t sgn = (L & M) ? 0x80000000u : 0u;
-#pragma unroll
-    for (int c = 0; c < 8; ++c) {
-        if constexpr (M == 4) {
-            const float up = __int_as_float(dpp_mov<0x104>(__float_as_int(x[c])));
-            const float dn = __int_as_float(dpp_mov<0x114>(__float_as_int(x[c])));
-            x[c] = (L & M) ? dn - x[c] : x[c] + up;
-        } else {
-            const float o = __int_as_float(dpp_mov<xor_dpp_ctrl<M>()>(__float_as_int(x[c])));
-            x[c] = o + __uint_as_float(__float_as_uint(x[c]) ^ sgn);
-        }
+// A butterfly gives the lane with bit M of L clear x + o and the other o - x (o the partner's value). Computed is x + o
+// and x - o, one fused multiply-add with the factor +-1 (exact, so only the sum rounds) that reads the partner's value by
+// DPP: one instruction a value. The lanes with the bit set then hold the negative; both partners of every later butterfly
+// hold the same sign, the butterfly is linear and rounding is symmetric, so the sign is the parity of L's bits at the end
+// and goes into the final factor. (Written as asm: the compiler keeps the DPP move and the fma apart. A DPP operand is read
+// at the earliest two wait states after it was written: the leading s_nop covers what the compiler wrote last, inside the
+// sequence eight instructions lie between. Every lane of the wave runs it.)
+// The prep is bound by VALU issue. With these, the mirrored quads (4 instructions a value for the butterflies over lane
+// bits, 9 with a sign flip and two-way shifts) and rn_byte (one in place of three): fused rmsRope + prep of 5,967 tokens x
+// 56 heads 161.4 -> 150.4 us, 4,000 x 32 70.8 -> 65.0, 1,000 x 24 25.8 -> 24.3; the call at head dim 64, 1,797 x 32,
+// 56.7 -> 55.6. The same bits.
+#define LR_I8_BUTTERFLY(s, ctrl)                     \
+    "v_fmac_f32_dpp %0, %0, " s " " ctrl "\n\t"      \
+    "v_fmac_f32_dpp %1, %1, " s " " ctrl "\n\t"      \
+    "v_fmac_f32_dpp %2, %2, " s " " ctrl "\n\t"      \
+    "v_fmac_f32_dpp %3, %3, " s " " ctrl "\n\t"      \
+    "v_fmac_f32_dpp %4, %4, " s " " ctrl "\n\t"      \
+    "v_fmac_f32_dpp %5, %5, " s " " ctrl "\n\t"      \
+    "v_fmac_f32_dpp %6, %6, " s " " ctrl "\n\t"      \
+    "v_fmac_f32_dpp %7, %7, " s " " ctrl "\n\t"
+#define LR_I8_BUTTERFLIES_124                                                          \
+    "s_nop 1\n\t" LR_I8_BUTTERFLY("%8", "quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf") \
+    LR_I8_BUTTERFLY("%9", "quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf")            \
+    LR_I8_BUTTERFLY("%10", "row_half_mirror row_mask:0xf bank_mask:0xf")
+#define LR_I8_X8 "+v"(x[0]), "+v"(x[1]), "+v"(x[2]), "+v"(x[3]), "+v"(x[4]), "+v"(x[5]), "+v"(x[6]), "+v"(x[7])
+template <int ROT>
+__device__ __forceinline__ void butterflies8(float (&x)[8], int L) {
+    const float s1 = (L & 1) ? -1.0f : 1.0f, s2 = (L & 2) ? -1.0f : 1.0f, s4 = (L & 4) ? -1.0f : 1.0f;
+    if constexpr (ROT == 128) {
+        const float s8 = (L & 8) ? -1.0f : 1.0f;
+        asm volatile(LR_I8_BUTTERFLIES_124 LR_I8_BUTTERFLY("%11", "row_ror:8 row_mask:0xf bank_mask:0xf")
+                     : LR_I8_X8 : "v"(s1), "v"(s2), "v"(s4), "v"(s8));
+    } else {
+        asm volatile(LR_I8_BUTTERFLIES_124 : LR_I8_X8 : "v"(s1), "v"(s2), "v"(s4));
     }
 }
 
@@ -182,25 +182,26 @@ __device__ __forceinline__ void rotate8(float (&x)[8], int L) {
     for (int g = 0; g < 2; ++g) {
         float* y = x + 4 * g;
         const float a0 = y[0] + y[1], a1 = y[0] - y[1], a2 = y[2] + y[3], a3 = y[2] - y[3];
-        y[0] = (a0 + a2) * 0.5f;
-        y[1] = (a1 + a3) * 0.5f;
-        y[2] = (a0 - a2) * 0.5f;
-        y[3] = (a1 - a3) * 0.5f;
+        y[0] = a0 + a2;   // * 0.5 below
+        y[1] = a1 + a3;
+        y[2] = a0 - a2;
+        y[3] = a1 - a3;
     }
     if (ROT == 128 || ROT == 64) {
 #pragma unroll
         for (int c = 0; c < 4; ++c) {  // lane bit 1: reference lane 2L adds, lane 2L + 1 subtracts its own value
-            const float e = x[c], o = x[4 + c];
-            x[c] = e + o;
-            x[4 + c] = e - o;
+            const float e = x[c], o = x[4 + c] * 0.5f;   // (e * 0.5 is exact: the fma's rounding is that of the sum)
+            x[c] = fmaf(e, 0.5f, o);
+            x[4 + c] = fmaf(e, 0.5f, -o);
         }
-        butterfly8<1>(x, L);
-        butterfly8<2>(x, L);
-        butterfly8<4>(x, L);
-        if (ROT == 128) butterfly8<8>(x, L);
+        butterflies8<ROT>(x, L);
         const float norm = ROT == 128 ? 0.1767766952966369f : 0.25f;
+        const float f = __popc(L & (ROT == 128 ? 15 : 7)) & 1 ? -norm : norm;
 #pragma unroll
-        for (int c = 0; c < 8; ++c) x[c] *= norm;
+        for (int c = 0; c < 8; ++c) x[c] *= f;
+    } else {
+#pragma unroll
+        for (int c = 0; c < 8; ++c) x[c] *= 0.5f;
     }
 }
 
@@ -213,18 +214,18 @@ __device__ __forceinline__ void load8(const uint16_t* p, float (&x)[8]) {
     }
 }
 
-// 8 values * inv, rounded and saturated to int8, as two little-endian words
+// 8 values * inv, rounded to int8 (rn_byte), as two little-endian words
 __device__ __forceinline__ u32x2 pack_s8x8(const float (&x)[8], float inv) {
 #pragma clang fp contract(off)
     int q[8];
 #pragma unroll
-    for (int c = 0; c < 8; ++c) q[c] = rn_sat(x[c] * inv);
+    for (int c = 0; c < 8; ++c) q[c] = rn_byte(x[c] * inv);
     return u32x2{pack_lo_bytes(q[0], q[1], q[2], q[3]), pack_lo_bytes(q[4], q[5], q[6], q[7])};
 }
 
 // ------------------------------------------------------------------------------------------------ fused rmsRope
 // Kitchen.rmsRope (kernels/cuda/minimax/kitchen/rms_rope.cu:37-230, as src/engines/minimax_h3/launch.zig:421-441
-// launches it) of one row held by a group of 16 lanes, lane L holding channels 8 L .. 8 L + 7, for the prep of
+// launches it) of one row held by a group of 16 lanes, lane group_lane(L) holding channels 8 L .. 8 L + 7, for the prep of
 // lr_int8_attention_prep_rope:
 //   rrms = 1 / sqrt(sum(x^2) / 128 + eps) and x * rrms * w, in double, rounded to fp32 and then to bf16 (the
 //   normalised value the reference rounds before the rotation, rms_rope.cu:143-150);
@@ -311,7 +312,7 @@ __device__ __forceinline__ void h3_rms_rope(float (&x)[8], int L, const float (&
     norm_bf16_exact8(x, rr, w);
     const int hc = rot >> 4;
     const bool first = L < hc, second = L >= hc && L < 2 * hc;
-    const int partner = first ? L + hc : (second ? L - hc : L);
+    const int partner = group_lane(first ? L + hc : (second ? L - hc : L));
     // first half: f00 x_i + f01 x_{i+rot/2} (own value x_i); second half: f10 x_i + f11 x_{i+rot/2} (own value
     // x_{i+rot/2}): with the second half's (f10, f11) swapped once, both are (own coefficient) * own + (partner's
     // coefficient) * partner. Both products are exact (bf16 times bf16), so the one rounding of the fma is the exact
@@ -383,7 +384,7 @@ __global__ __launch_bounds__(256) void i8_stats_kernel(PrepArgs a) {
     // prepares every key row
     float (*rows)[128] = reinterpret_cast<float (*)[128]>(smem + SD_BYTES);
     if constexpr (ROPE) {
-        const int grp = t >> 4, L = t & 15;
+        const int grp = t >> 4, L = group_lane(t & 15);
         if (grp < NSAMP) {
             const int row = (int)((int64_t)grp * (a.Sk - 1) / (NSAMP - 1));
             float x[8], wv[8];
@@ -479,7 +480,7 @@ __device__ void quant_q(const PrepArgs& a, int b, int h, int qb, uint8_t* lds) {
 #pragma clang fp contract(off)
     constexpr int LPR = HD / 8, RPB = 256 / LPR, NR = QROWS / RPB;  // lanes a row, rows a block pass, rows a lane
     const Plan& p = a.p;
-    const int t = threadIdx.x, slot = t / LPR, L = t % LPR;
+    const int t = threadIdx.x, slot = t / LPR, L = group_lane(t % LPR);
     const uint16_t* qbase = a.q + b * a.q_sb + h * a.q_sh + 8 * L;
     if constexpr (ROPE) rope_tab_dma(a, lds, [&](int r) { return min(qb * QROWS + r, a.Sq - 1); });
     u32x4 raw[NR];
@@ -537,7 +538,7 @@ __device__ void quant_k(const PrepArgs& a, int b, int hk, int kb, uint8_t* lds) 
     static_assert(NPASS % 2 == 0 && KGROUP % RPW == 0, "passes run in pairs; a wave's rows lie in one group");
     __shared__ float gmax[KROWS / KGROUP][4];   // [group][wave within the group]
     const Plan& p = a.p;
-    const int t = threadIdx.x, wave = t >> 6, prow = t / LPR, L = t % LPR;
+    const int t = threadIdx.x, wave = t >> 6, prow = t / LPR, L = group_lane(t % LPR);
     const uint16_t* kbase = a.k + b * a.k_sb + hk * a.k_sh + 8 * L;
     // Rows past Sk (the last tile's padding) repeat real keys: those of the last key's scale group gL, key Sk - 1
     // standing in past its end. A padded row of group gL then equals key Sk - 1 and leaves the group's scale as it
@@ -644,8 +645,8 @@ __device__ void quant_v(const PrepArgs& a, int b, int hk, int tile, uint8_t* ext
             int lo[4], hi[4];
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                lo[r] = rn_sat(lo_bf16(raw[r][j]) * inv[2 * j]);
-                hi[r] = rn_sat(hi_bf16(raw[r][j]) * inv[2 * j + 1]);
+                lo[r] = rn_byte(lo_bf16(raw[r][j]) * inv[2 * j]);
+                hi[r] = rn_byte(hi_bf16(raw[r][j]) * inv[2 * j + 1]);
             }
             col[2 * j] = pack_lo_bytes(lo[0], lo[1], lo[2], lo[3]);
             col[2 * j + 1] = pack_lo_bytes(hi[0], hi[1], hi[2], hi[3]);
