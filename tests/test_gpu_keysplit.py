@@ -126,3 +126,17 @@ def test_keysplit_images_against_the_streaming_kernel(Sq, Sk, H, HK):
                 for c in (ops.CFG_AUTO, ops.CFG_STREAM_W8))
     torch.cuda.synchronize()
     assert_close(got, bf16_f32(ref).astype(np.float64), rel=6e-3, what="images")
+
+
+def test_keysplit_row_of_one_key_is_its_value():
+    """A row that sees one key returns that key's value to the bit: the probabilities are normalised by the sum of their
+    rounded values, so the one factor left is p * (1 / p) in fp32, far below a bf16 rounding. Over rows the first row of a
+    causal call (its second group of waves sees no key), over images a call of one key."""
+    W, H = 600, 3
+    q, k, v = _qkv(76, W, W, H, H)
+    dq, dk, dv = to_dev(q), to_dev(k), to_dev(v)
+    got = from_dev(ops.attention(dq, dk, dv, causal=True))
+    assert np.array_equal(got[0], from_dev(dv)[0])
+    got = from_dev(ops.joint_attention(dq, dk[:1].contiguous(), dv[:1].contiguous(), table_kind=0))
+    torch.cuda.synchronize()
+    assert np.array_equal(got, np.broadcast_to(from_dev(dv)[:1], got.shape))
