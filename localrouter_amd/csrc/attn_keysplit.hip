@@ -231,11 +231,10 @@ __global__ __launch_bounds__(512, 1) __attribute__((amdgpu_waves_per_eu(2, 2))) 
         }
     };
 
-    // ---- the queries and K(0) resident; S of the group's first half-tile and the fixed reference m = ceil(max) (exp2
-    // domain, held as m / c; see attn_stream.hip). A row with no key in it (causal) keeps m = 0 and P = 0.
+    // ---- the queries and K(0) resident; S of the group's first half-tile and the fixed reference m = its maximum. A row with
+    // no key in it (causal) keeps m = 0 and P = 0.
 #pragma unroll
     for (int db = 0; db < 4; ++db) o[db] = f32x16{};
-    const float rc = 1.0f / c;
     LR_WAIT_VMCNT(0);
     block_barrier();
     {
@@ -262,11 +261,13 @@ __global__ __launch_bounds__(512, 1) __attribute__((amdgpu_waves_per_eu(2, 2))) 
 #pragma unroll
         for (int q = 1; q < 16; ++q) mx = fmaxf(mx, s[0][q]);
         mx = wave_pair_max(mx);
-        mref = mx > -INFINITY ? ceilf(mx * c) : 0.0f;
-        float mc = mref * rc;   // (its rounding shifts every exponent of the row alike, so it is rounded once: opaque, or
-        asm volatile("" : "+v"(mc));   // the subtraction below could take the product unrounded)
-        negm = f32x16{} - mc;
-        s[0] -= mc;
+        // (the maximum itself, not the next integer: where it is the row's, its probability is 1, with no rounding of its
+        // own. Relative error against 64 bits of causal calls, 500 queries x 16 heads 2.12e-3 -> 2.00e-3, 4,000 x 24 2.18e-3 ->
+        // 2.09e-3, as the pipelined kernel's; the same time)
+        const float m0 = mx > -INFINITY ? mx : 0.0f;
+        mref = m0 * c;
+        negm = f32x16{} - m0;
+        s[0] -= m0;
         asm volatile(LR_NOP48 : "+v"(negm));
     }
     // ---- step 0: S of half-tile 1 (K(0), fragments 8-15), P of half-tile 0

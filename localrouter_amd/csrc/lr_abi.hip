@@ -98,6 +98,8 @@ bool keysplit_fits(int W, int H, int nkeys, int cus, bool split_area) {
 // merge), so calls of fewer than 8 key tiles keep it (320 x 4 heads 11.7 / 10.4 us, 256 x 24 10.6 / 9.8). Causal calls
 // take the key-split kernel whatever their size: its blocks run longest first and each in half the steps (1,500 queries
 // x 1,577 keys, 32 heads over 8, 32.7 / 40.4 us; 2,048 42.7 / 57.8; 4,096 140 / 187; 4,608 x 24 142 / 178).
+// (All taken before the key-split kernel summed its rounded probabilities, which adds 1 to 3 % to its side: 600 x 16 15.8 us,
+// 1,000 queries x 1,500 keys x 24 heads 30.0 / 33.0, 300 x 3,000 x 16 42.8 / 53.5, causal 500 x 16 13.8 / 15.2.)
 bool keysplit_rows(int W, int H, int nkeys, int causal, int cus, bool split_area) {
     if (nkeys <= 7 * 64 || cus < 1) return false;
     const int64_t blocks = (int64_t)((W + 127) / 128) * H;
