@@ -172,7 +172,7 @@ def test_int8_packed_qkv(S, H, bias):
 
 def test_int8_prep_nonfinite_values():
     """NaN and infinities in q, k and v: the quantisers' NaN -> 0 and saturation (float_utils.cuh:40-51; the
-    kernels convert through v_cvt_i32_f32, which maps NaN to 0 and saturates), the abs-max that skips NaN (fmaxf),
+    kernels round by an add whose low byte a NaN leaves 0), the abs-max that skips NaN (fmaxf),
     and the infinite scales: the prep still bit-exact against the oracle. The planted rows are not anchor samples."""
     S, H = 300, 2
     print(f"\n[int8 non-finite] S={S} H={H}", flush=True)
