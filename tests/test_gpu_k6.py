@@ -122,3 +122,26 @@ def test_key_split_attention(W, S, H, HK):
     dp = np.abs(_f32(out) - _f32(plain))
     mx, mn = assert_close(_bits(out), ref, what=f"key split {W}x{S}x{H}/{HK}")
     print(f"  max-abs {mx:.3e} mean-abs {mn:.3e}; vs unsplit max {dp.max():.3e}", flush=True)
+
+
+@pytest.mark.parametrize("bad", [float("inf"), float("nan")])
+def test_key_split_keeps_nonfinite_values_of_a_negligible_range(bad):
+    """A value of infinity or NaN in a key range whose weight underflows to 0 beside another range's: 0 times it is NaN, in
+    the merge of the ranges as in the unsplit call. Every query is ones, every key zeros but for key 5, which is tens: its
+    score lies 163 (exp2 domain) above the others', below 2^-149. The value is planted in dim 7 of key 3,000."""
+    from localrouter_amd import _lib, ops
+    W, S, H = 40, 4096, 2
+    print(f"key split, planted value {bad}", flush=True)
+    assert int(_lib.load().lr_attention_ws_bytes(W, H, S, 0)) > 0
+    q = torch.ones(W, H, 128, dtype=torch.bfloat16, device="cuda")
+    k = torch.zeros(S, H, 128, dtype=torch.bfloat16, device="cuda")
+    k[5] = 10.0
+    v = _rand((S, H, 128), torch.Generator(device="cuda").manual_seed(9), "cuda")
+    v[3000, :, 7] = bad
+    out, plain = ops.attention_ws(q, k, v, scale=SCALE), ops.attention(q, k, v, scale=SCALE)
+    torch.cuda.synchronize()
+    want = torch.zeros(128, dtype=torch.bool, device="cuda")
+    want[7] = True
+    assert torch.equal(plain.isnan(), want.expand(W, H, 128))
+    assert torch.equal(out.isnan(), want.expand(W, H, 128))
+    assert torch.equal(out[..., ~want], v[5][:, ~want].expand(W, H, 127))
