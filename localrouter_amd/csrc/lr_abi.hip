@@ -111,6 +111,29 @@ bool keysplit_rows(int W, int H, int nkeys, int causal, int cus, bool split_area
     return causal || keysplit_fits(W, H, nkeys, cus, split_area);
 }
 
+// The kernel of a call over key and value rows under LR_ATTN_CFG_AUTO. ranges: the call can be split over the keys
+// (split_count, and its workspace holds the partials); split_area: its workspace holds the streaming kernel's split area;
+// narrow: its strides suit the kernels that take 32-bit per-lane row offsets (wider ones go on to the pipelined kernels).
+// Up to 24 key tiles the key-split kernel is as fast as the split over workgroups and its merge launch (500 queries x 1,100
+// keys x 16 heads 20.7 / 30.0 us, 150 x 1,000 x 32 19.1 / 22.9, 218 x 1,500 x 16 24.4 / 24.6; 2,500 keys 35.0 / 27.3).
+int rows_route(int W, int H, int nkeys, int causal, int cus, bool ranges, bool split_area, bool narrow) {
+    const bool keysplit = narrow && keysplit_rows(W, H, nkeys, causal, cus, split_area);
+    if (ranges && !(keysplit && nkeys <= 24 * 64)) return lr::ROUTE_KEY_RANGES;
+    if (keysplit) return lr::ROUTE_KEYSPLIT;
+    if (stream_rows(W, H, nkeys, causal, split_area, cus)) return lr::ROUTE_STREAM;
+    // 128 queries per workgroup, two workgroups per CU, unless non-causal 256-query blocks fill whole rounds of
+    // the CUs: measured at cfg1 / cfg2 / causal GQA shapes W4 takes 0.72 / 0.93 / 0.89 of W8's time, at 12,800
+    // and 50,220 tokens the two are within 1.5 %, at 16,384 x 4 heads (exactly one round of 256-query blocks) W8
+    // is 2 % faster; causal blocks differ in work, and W4 stays faster there even when the rounds are whole
+    const int64_t w8_blocks = (int64_t)((W + 255) / 256) * H;
+    return !causal && cus > 0 && w8_blocks % cus == 0 ? lr::ROUTE_PIPE_W8 : lr::ROUTE_PIPE_W4;
+}
+
+// The kernel of the attention over key tile images (the fused, prepared and stage calls).
+int images_route(int W, int H, int nkeys, int causal, int cus) {
+    return !causal && keysplit_fits(W, H, nkeys, cus, true) ? lr::ROUTE_KEYSPLIT : lr::ROUTE_STREAM;
+}
+
 size_t split_bytes(int W, int H, int ns) {
     if (ns <= 1) return 0;
     const size_t rows = (size_t)H * W * ns;
@@ -142,16 +165,13 @@ int attention_impl(const void* q, const void* k, const void* v, void* out, int p
     const int ns = split_count(W, H, nkeys, causal);
     const int cus = config == LR_ATTN_CFG_AUTO || config == LR_ATTN_CFG_STREAM_W8 ? device_cus() : 0;
     const bool ws_split_area = workspace && ws_bytes >= (size_t)LR_JOINT_SPLIT_BYTES && aligned(workspace, 256);
-    // (the key-split kernel takes 32-bit per-lane row offsets, as the streaming kernel does: wider strides go on)
-    const bool keysplit = config == LR_ATTN_CFG_AUTO && keysplit_rows(W, H, nkeys, causal, cus, ws_split_area) &&
-                          k_rs <= lr::STREAM_MAX_V_RS && v_rs <= lr::STREAM_MAX_V_RS;
-    // up to 24 key tiles the key-split kernel is as fast as the split over workgroups and its merge launch (500 queries x
-    // 1,100 keys x 16 heads 20.7 / 30.0 us, 150 x 1,000 x 32 19.1 / 22.9, 218 x 1,500 x 16 24.4 / 24.6; 2,500 keys 35.0 /
-    // 27.3)
-    const bool split = workspace && ns > 1 && (config == LR_ATTN_CFG_AUTO || config == LR_ATTN_CFG_PIPE_W8) &&
-                       !(keysplit && nkeys <= 24 * 64) && k_hs == lr::D && v_hs == lr::D &&
-                       ws_bytes >= split_bytes(W, H, ns) && aligned(workspace, 256);
-    if (split) {
+    const bool ranges = workspace && ns > 1 && k_hs == lr::D && v_hs == lr::D && ws_bytes >= split_bytes(W, H, ns) &&
+                        aligned(workspace, 256);
+    const bool narrow = k_rs <= lr::STREAM_MAX_V_RS && v_rs <= lr::STREAM_MAX_V_RS;
+    int route = config;
+    if (config == LR_ATTN_CFG_AUTO) route = rows_route(W, H, nkeys, causal, cus, ranges, ws_split_area, narrow);
+    else if (config == LR_ATTN_CFG_PIPE_W8 && ranges) route = lr::ROUTE_KEY_RANGES;
+    if (route == lr::ROUTE_KEY_RANGES) {
         a.nsplit = ns;
         a.part_o = static_cast<float*>(workspace);
         a.part_ml = reinterpret_cast<float*>(static_cast<char*>(workspace) +
@@ -160,18 +180,8 @@ int attention_impl(const void* q, const void* k, const void* v, void* out, int p
         if (e != hipSuccess) return (int)e;
         return (int)lr::launch_split_combine(a, stream);
     }
-    if (keysplit) return (int)lr::launch_keysplit(a, stream, true);
-    if (config == LR_ATTN_CFG_AUTO && stream_rows(W, H, nkeys, causal, ws_split_area, cus)) {
-        config = LR_ATTN_CFG_STREAM_W8;
-    } else if (config == LR_ATTN_CFG_AUTO) {
-        // 128 queries per workgroup, two workgroups per CU, unless non-causal 256-query blocks fill whole rounds of
-        // the CUs: measured at cfg1 / cfg2 / causal GQA shapes W4 takes 0.72 / 0.93 / 0.89 of W8's time, at 12,800
-        // and 50,220 tokens the two are within 1.5 %, at 16,384 x 4 heads (exactly one round of 256-query blocks) W8
-        // is 2 % faster; causal blocks differ in work, and W4 stays faster there even when the rounds are whole
-        const int64_t w8_blocks = (int64_t)((W + 255) / 256) * H;
-        config = !causal && cus > 0 && w8_blocks % cus == 0 ? LR_ATTN_CFG_PIPE_W8 : LR_ATTN_CFG_PIPE_W4;
-    }
-    if (config == LR_ATTN_CFG_STREAM_W8) {
+    if (route == lr::ROUTE_KEYSPLIT) return (int)lr::launch_keysplit(a, stream, true);
+    if (route == lr::ROUTE_STREAM) {
         // the streaming kernel over the key rows: the output's 32-bit buffer range (256 rows * o_rs * 2 bytes < 2^32)
         // and 32-bit per-lane row offsets (k_rs, v_rs <= STREAM_MAX_V_RS); with a workspace, its split tail
         if (o_rs >= ((int64_t)1 << 23) || k_rs > lr::STREAM_MAX_V_RS || v_rs > lr::STREAM_MAX_V_RS) return ERR_ARGS;
@@ -183,7 +193,7 @@ int attention_impl(const void* q, const void* k, const void* v, void* out, int p
         }
         return (int)lr::launch_stream(a, nwg, stream, true);
     }
-    return (int)lr::launch_attention(a, config, stream);
+    return (int)lr::launch_attention(a, route, stream);
 }
 
 // Table checks shared by the rope entry points. rows_needed: table rows that will be read.
@@ -388,7 +398,7 @@ int images_launch(const void* q_prep, int64_t p_rs, const void* ws, void* out, i
     char* split = split_area(const_cast<void*>(ws), Sk, HK);
     a.part = split;
     a.cnt = reinterpret_cast<int*>(split + lr::STREAM_PART_BYTES);
-    if (config == LR_ATTN_CFG_AUTO && !causal && keysplit_fits(Sq, H, Sk, cus, true))
+    if (config == LR_ATTN_CFG_AUTO && images_route(Sq, H, Sk, causal, cus) == lr::ROUTE_KEYSPLIT)
         return (int)lr::launch_keysplit(a, stream, false);
     return (int)lr::launch_stream(a, cus, stream);
 }
@@ -594,6 +604,14 @@ void* device_scratch(int* err) {
 extern "C" {
 
 int lr_attn_abi_version(void) { return LR_ATTN_ABI_VERSION; }
+
+int lr_attention_route(int W, int H, int HK, int nkeys, int causal, int p0, size_t workspace_bytes, int images, int cus) {
+    if (W < 1 || H < 1 || HK < 1 || nkeys < 1 || p0 < 0) return 0;
+    if (images) return images_route(W, H, nkeys, causal, std::min(cus, lr::STREAM_MAX_WG));
+    const int ns = split_count(W, H, nkeys, causal);
+    return rows_route(W, H, nkeys, causal, cus, ns > 1 && workspace_bytes >= split_bytes(W, H, ns),
+                      workspace_bytes >= (size_t)LR_JOINT_SPLIT_BYTES, true);
+}
 
 int lr_attn_init(void) {
     int dev = 0;

@@ -60,6 +60,15 @@ enum AttnConfig : int {
     ATTN_CFG_STREAM_W8 = 9,    // fused / prepared calls: the persistent streaming kernel over tile images
 };
 
+// The kernel a call takes under LR_ATTN_CFG_AUTO: one of the configurations, or a kernel that no configuration names.
+enum AttnRoute : int {
+    ROUTE_PIPE_W8 = ATTN_CFG_PIPE_W8,
+    ROUTE_PIPE_W4 = ATTN_CFG_PIPE_W4,
+    ROUTE_STREAM = ATTN_CFG_STREAM_W8,
+    ROUTE_KEY_RANGES = 32,   // the 256-query pipelined kernel over ranges of the keys, then the merge
+    ROUTE_KEYSPLIT = 33,     // attn_keysplit.hip
+};
+
 // Plain attention over value rows (AUTO = PIPE_W8; a.nsplit > 1 splits every query block over the keys).
 hipError_t launch_attention(const AttnArgs& a, int config, hipStream_t stream);
 // keys.hip: gather the kept keys (kmask[j] != 0, in order) and their value rows into kc / vc [n_valid][HK * 128], one
@@ -117,3 +126,9 @@ constexpr int64_t STREAM_PART_BYTES = 2 * STREAM_MAX_WG * STREAM_SLOT_BYTES;
 constexpr int64_t STREAM_CNT_BYTES = 4 * STREAM_MAX_WG;                 // arrival counters (one per cut block)
 
 }  // namespace lr
+
+// The AttnRoute of a call under LR_ATTN_CFG_AUTO on a device of cus compute units (host arithmetic only; 0: sizes no call
+// takes). images: the fused, prepared and stage calls; else key and value rows, workspace_bytes of scratch (0: none).
+// Exported beside the ABI of include/, for the tests of the rules and so that a kernel's tests can assert that it runs.
+extern "C" int lr_attention_route(int W, int H, int HK, int nkeys, int causal, int p0, size_t workspace_bytes, int images,
+                                  int cus);

@@ -74,3 +74,21 @@ def decode_images(raw: np.ndarray, Sk: int, HK: int):
     keys = kimg[:, :, img_index()].reshape(HK, nt * 64, 128)
     vals = u[HK * nt * 8192:].reshape(nt * 64, HK, 128).transpose(1, 0, 2)
     return keys, vals
+
+
+# ------------------------------------------------------------------------------------------ routes
+PIPE_W8, PIPE_W4, STREAM, KEY_RANGES, KEYSPLIT = 1, 2, 9, 32, 33   # AttnRoute, csrc/lr_kernels.h
+
+
+def route(W: int, H: int, nkeys: int, HK: int | None = None, causal: int = 0, p0: int = 0, workspace: bool = False,
+          images: bool = False, cus: int = 256) -> int:
+    """The kernel that LR_ATTN_CFG_AUTO takes for a call of these sizes. workspace: lr_attention_bf16_ws with the bytes
+    lr_attention_ws_bytes asks for."""
+    import ctypes
+
+    from localrouter_amd import _lib
+    L = _lib.load()
+    fn = L.lr_attention_route
+    fn.restype, fn.argtypes = ctypes.c_int, [ctypes.c_int] * 6 + [ctypes.c_size_t] + [ctypes.c_int] * 2
+    nb = int(L.lr_attention_ws_bytes(W, H, nkeys, causal)) if workspace else 0
+    return fn(W, H, H if HK is None else HK, nkeys, causal, p0, nb, int(images), cus)

@@ -1,0 +1,34 @@
+"""Which kernel a call's sizes lead to (localrouter_amd/csrc/lr_abi.hip, through lr_attention_route: host arithmetic, no GPU),
+on 256 compute units: the lines the rules draw, from both sides."""
+from __future__ import annotations
+
+import pytest
+
+from tests._util import KEY_RANGES, KEYSPLIT, PIPE_W4, PIPE_W8, STREAM, route
+
+
+def test_sizes_no_call_takes():
+    for bad in (dict(W=0), dict(H=0), dict(HK=0), dict(nkeys=0), dict(p0=-1)):
+        assert route(**{**dict(W=8, H=2, nkeys=8), **bad}) == 0
+
+
+@pytest.mark.parametrize("W,H,nkeys,want", [
+    (1280, 24, 1280, KEYSPLIT),      # 240 blocks of 128 queries: one round
+    (2000, 24, 2000, PIPE_W4),       # 384: past one round
+    (16384, 4, 2000, PIPE_W8),       # 256 blocks of 256 queries
+    (4608, 24, 4608, STREAM),        # from 4,096 keys on, 432 blocks of 256 queries
+    (320, 24, 320, PIPE_W4),         # too few key tiles for the key-split kernel's longer start
+])
+def test_rows(W, H, nkeys, want):
+    assert route(W, H, nkeys) == want
+
+
+@pytest.mark.parametrize("W,H,nkeys,want", [(218, 16, 50220, KEY_RANGES), (4608, 24, 4608, STREAM), (218, 16, 300, PIPE_W4)])
+def test_rows_with_a_workspace(W, H, nkeys, want):
+    assert route(W, H, nkeys, workspace=True) == want
+
+
+@pytest.mark.parametrize("Sq,H,Sk,want", [(320, 4, 320, KEYSPLIT), (1280, 24, 1280, KEYSPLIT), (4608, 24, 4608, STREAM)])
+def test_images(Sq, H, Sk, want):
+    assert route(Sq, H, Sk, images=True) == want
+    assert route(Sq, H, Sk, images=True, causal=1) == STREAM
