@@ -100,7 +100,10 @@ bool keysplit_fits(int W, int H, int nkeys, int cus, bool split_area) {
 // x 1,577 keys, 32 heads over 8, 32.7 / 40.4 us; 2,048 42.7 / 57.8; 4,096 140 / 187; 4,608 x 24 142 / 178).
 // (All taken before the key-split kernel summed its rounded probabilities, which adds 1 to 3 % to its side: 600 x 16 15.8 us,
 // 1,000 queries x 1,500 keys x 24 heads 30.0 / 33.0, 300 x 3,000 x 16 42.8 / 53.5, causal 500 x 16 13.8 / 15.2.)
-bool keysplit_rows(int W, int H, int nkeys, int causal, int cus, bool split_area) {
+// What counts are the keys that some row sees: a causal chunk at the front of a longer key buffer is a short call (64 queries at
+// position 0 x 16 heads 8.0 us by the key-split kernel, 6.8 by the pipelined one; one query 7.3 and 5.7).
+bool keysplit_rows(int W, int H, int all_keys, int causal, int p0, int cus, bool split_area) {
+    const int nkeys = causal ? (int)std::min<int64_t>(all_keys, (int64_t)p0 + W) : all_keys;
     if (nkeys <= 7 * 64 || cus < 1) return false;
     const int64_t blocks = (int64_t)((W + 127) / 128) * H;
     if (blocks > 1 << 22) return false;   // (a grid's work-items are counted in 32 bits)
@@ -116,8 +119,8 @@ bool keysplit_rows(int W, int H, int nkeys, int causal, int cus, bool split_area
 // narrow: its strides suit the kernels that take 32-bit per-lane row offsets (wider ones go on to the pipelined kernels).
 // Up to 24 key tiles the key-split kernel is as fast as the split over workgroups and its merge launch (500 queries x 1,100
 // keys x 16 heads 20.7 / 30.0 us, 150 x 1,000 x 32 19.1 / 22.9, 218 x 1,500 x 16 24.4 / 24.6; 2,500 keys 35.0 / 27.3).
-int rows_route(int W, int H, int nkeys, int causal, int cus, bool ranges, bool split_area, bool narrow) {
-    const bool keysplit = narrow && keysplit_rows(W, H, nkeys, causal, cus, split_area);
+int rows_route(int W, int H, int nkeys, int causal, int p0, int cus, bool ranges, bool split_area, bool narrow) {
+    const bool keysplit = narrow && keysplit_rows(W, H, nkeys, causal, p0, cus, split_area);
     if (ranges && !(keysplit && nkeys <= 24 * 64)) return lr::ROUTE_KEY_RANGES;
     if (keysplit) return lr::ROUTE_KEYSPLIT;
     if (stream_rows(W, H, nkeys, causal, split_area, cus)) return lr::ROUTE_STREAM;
@@ -169,7 +172,7 @@ int attention_impl(const void* q, const void* k, const void* v, void* out, int p
                         aligned(workspace, 256);
     const bool narrow = k_rs <= lr::STREAM_MAX_V_RS && v_rs <= lr::STREAM_MAX_V_RS;
     int route = config;
-    if (config == LR_ATTN_CFG_AUTO) route = rows_route(W, H, nkeys, causal, cus, ranges, ws_split_area, narrow);
+    if (config == LR_ATTN_CFG_AUTO) route = rows_route(W, H, nkeys, causal, p0, cus, ranges, ws_split_area, narrow);
     else if (config == LR_ATTN_CFG_PIPE_W8 && ranges) route = lr::ROUTE_KEY_RANGES;
     if (route == lr::ROUTE_KEY_RANGES) {
         a.nsplit = ns;
@@ -609,7 +612,7 @@ int lr_attention_route(int W, int H, int HK, int nkeys, int causal, int p0, size
     if (W < 1 || H < 1 || HK < 1 || nkeys < 1 || p0 < 0) return 0;
     if (images) return images_route(W, H, nkeys, causal, std::min(cus, lr::STREAM_MAX_WG));
     const int ns = split_count(W, H, nkeys, causal);
-    return rows_route(W, H, nkeys, causal, cus, ns > 1 && workspace_bytes >= split_bytes(W, H, ns),
+    return rows_route(W, H, nkeys, causal, p0, cus, ns > 1 && workspace_bytes >= split_bytes(W, H, ns),
                       workspace_bytes >= (size_t)LR_JOINT_SPLIT_BYTES, true);
 }
 

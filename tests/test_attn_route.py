@@ -28,6 +28,15 @@ def test_rows_with_a_workspace(W, H, nkeys, want):
     assert route(W, H, nkeys, workspace=True) == want
 
 
+@pytest.mark.parametrize("W,p0,want", [(100, 0, PIPE_W4), (448, 0, PIPE_W4), (128, 320, PIPE_W4), (449, 0, KEYSPLIT),
+                                       (128, 321, KEYSPLIT)])
+def test_causal_calls_count_the_keys_they_see(W, p0, want):
+    """A causal chunk sees p0 + W keys, however long the buffer behind them is."""
+    for nkeys in (p0 + W, 512, 3000, 100000):
+        if nkeys >= p0 + W:
+            assert route(W, 16, nkeys, causal=1, p0=p0) == want, nkeys
+
+
 @pytest.mark.parametrize("Sq,H,Sk,want", [(320, 4, 320, KEYSPLIT), (1280, 24, 1280, KEYSPLIT), (4608, 24, 4608, STREAM)])
 def test_images(Sq, H, Sk, want):
     assert route(Sq, H, Sk, images=True) == want
