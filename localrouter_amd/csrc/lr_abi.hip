@@ -76,25 +76,26 @@ bool stream_rows_split(int W, int H, int nkeys, int cus) {
     return !(nkeys > 16384 && 4 * tail >= 3 * (int64_t)cus);
 }
 
-// Whether a non-causal call runs the key-split kernel (attn_keysplit.hip: 128-query blocks, one workgroup each, two key
-// groups) in place of the streaming kernel (or, over rows, the pipelined kernels): its blocks fit one round of the CUs
-// and, where the streaming kernel could cut its tail (split_area), half the key tiles are no more than the tiles a
-// workgroup of that tail takes plus 12 (the ~16 us its partials, merges and longer start cost, at ~1.3 us a tile).
-// Measured (us, this kernel / the other): fused 320 x 4 heads 14.9 / 24.5, 512 x 24 18.8 / 30.9, 1,280 x 24 34.3 / 48.4,
-// 3,000 x 4 43.0 / 50.1; past one round it gains nothing (fused 1,600 x 24, 1.2 rounds, 59.9 / 60.5; 3,000 x 12, 1.1
-// rounds, 90.8 / 77.5; 4,608 x 24 263 / 248); over rows against the 128-query pipelined kernel 600 x 16 14.9 / 16.5,
-// 1,024 queries x 1,104 keys x 32 23.6 / 26.5, 1,280 x 24 26.1 / 27.2, and 2,000 x 24 (1.5 rounds) 69.6 / 60.3.
-bool keysplit_fits(int W, int H, int nkeys, int cus, bool split_area) {
+// Whether a non-causal call over tile images runs the key-split kernel (attn_keysplit.hip: 128-query blocks, one workgroup
+// each, two key groups) in place of the streaming kernel: its blocks fit one round of the CUs and, where the streaming
+// kernel would cut its tail, half the key tiles are no more than the tiles a workgroup of that tail takes plus 12 (the
+// ~16 us its partials, merges and longer start cost, at ~1.3 us a tile).
+// Measured (us, this kernel / the other): 320 x 4 heads 14.9 / 24.5, 512 x 24 18.8 / 30.9, 1,280 x 24 34.3 / 48.4,
+// 3,000 x 4 43.0 / 50.1; past one round it gains nothing (1,600 x 24, 1.2 rounds, 59.9 / 60.5; 3,000 x 12, 1.1
+// rounds, 90.8 / 77.5; 4,608 x 24 263 / 248).
+bool keysplit_images(int W, int H, int nkeys, int cus) {
     const int64_t blocks = (int64_t)((W + 127) / 128) * H, T = (nkeys + 63) / 64;
     if (blocks > cus) return false;
     int tail_wg = 0;
     const int nwg = std::min(cus, lr::STREAM_MAX_WG);
-    if (!split_area || !lr::stream_split_params(W, H, nkeys, 0, nwg, &tail_wg)) return true;
+    if (!lr::stream_split_params(W, H, nkeys, 0, nwg, &tail_wg)) return true;
     const int64_t tail = (int64_t)((W + 255) / 256) * H % nwg;   // <= blocks <= cus: all of them when below nwg
     return (T + 1) / 2 <= (tail * T + tail_wg - 1) / tail_wg + 12;
 }
 
-// The same over key and value rows. The pipelined kernel starts sooner (~2.5 us: fewer loads before its first product, no
+// The same over key and value rows, for calls whose other kernel is a pipelined one (or, without scratch, the streaming
+// kernel's whole blocks): non-causal ones of at most one round of its blocks (600 x 16 heads 14.9 / 16.5 us, 1,024 queries x
+// 1,104 keys x 32 23.6 / 26.5, 1,280 x 24 26.1 / 27.2, and 2,000 x 24, 1.5 rounds, 69.6 / 60.3). The pipelined kernel starts sooner (~2.5 us: fewer loads before its first product, no
 // merge), so calls of fewer than 8 key tiles keep it (320 x 4 heads 11.7 / 10.4 us, 256 x 24 10.6 / 9.8). Causal calls
 // take the key-split kernel whatever their size: its blocks run longest first and each in half the steps (1,500 queries
 // x 1,577 keys, 32 heads over 8, 32.7 / 40.4 us; 2,048 42.7 / 57.8; 4,096 140 / 187; 4,608 x 24 142 / 178).
@@ -111,7 +112,7 @@ bool keysplit_rows(int W, int H, int all_keys, int causal, int p0, int cus, bool
     // better than the pipelined kernel's ring (64 queries x 32 heads, 4,096 / 32,768 keys 68 / 713 us against 64 / 635;
     // 128 x 4 heads, 8,192 / 16,384 keys 102 / 243 against 123 / 239; 500 x 16 heads, 32,768 keys 475 against 483)
     if ((causal || !split_area) && nkeys >= 4096 && (W <= 64 || (nkeys >= 16384 && blocks <= 32))) return false;
-    return causal || keysplit_fits(W, H, nkeys, cus, split_area);
+    return causal || blocks <= cus;
 }
 
 // The kernel of a call over key and value rows under LR_ATTN_CFG_AUTO. ranges: the call can be split over the keys
@@ -119,11 +120,16 @@ bool keysplit_rows(int W, int H, int all_keys, int causal, int p0, int cus, bool
 // narrow: its strides suit the kernels that take 32-bit per-lane row offsets (wider ones go on to the pipelined kernels).
 // Up to 24 key tiles the key-split kernel is as fast as the split over workgroups and its merge launch (500 queries x 1,100
 // keys x 16 heads 20.7 / 30.0 us, 150 x 1,000 x 32 19.1 / 22.9, 218 x 1,500 x 16 24.4 / 24.6; 2,500 keys 35.0 / 27.3).
+// With a split area the streaming kernel's tail puts all workgroups on the calls it takes: from 4,096 keys on the key-split
+// kernel is slower on them (streaming / key-split, us, keys and values not in the caches: 32 queries x 40 heads 52 / 98 and 84 /
+// 190 over 4,096 and 8,192 keys, 600 x 16 58 / 84 and 92 / 158, 2,048 x 16 79 / 85 and 134 / 156, 1,000 x 32 over 16,384
+// 244 / 327).
 int rows_route(int W, int H, int nkeys, int causal, int p0, int cus, bool ranges, bool split_area, bool narrow) {
-    const bool keysplit = narrow && keysplit_rows(W, H, nkeys, causal, p0, cus, split_area);
+    const bool stream = stream_rows(W, H, nkeys, causal, split_area, cus);
+    const bool keysplit = narrow && !(stream && split_area) && keysplit_rows(W, H, nkeys, causal, p0, cus, split_area);
     if (ranges && !(keysplit && nkeys <= 24 * 64)) return lr::ROUTE_KEY_RANGES;
     if (keysplit) return lr::ROUTE_KEYSPLIT;
-    if (stream_rows(W, H, nkeys, causal, split_area, cus)) return lr::ROUTE_STREAM;
+    if (stream) return lr::ROUTE_STREAM;
     // 128 queries per workgroup, two workgroups per CU, unless non-causal 256-query blocks fill whole rounds of
     // the CUs: measured at cfg1 / cfg2 / causal GQA shapes W4 takes 0.72 / 0.93 / 0.89 of W8's time, at 12,800
     // and 50,220 tokens the two are within 1.5 %, at 16,384 x 4 heads (exactly one round of 256-query blocks) W8
@@ -134,7 +140,7 @@ int rows_route(int W, int H, int nkeys, int causal, int p0, int cus, bool ranges
 
 // The kernel of the attention over key tile images (the fused, prepared and stage calls).
 int images_route(int W, int H, int nkeys, int causal, int cus) {
-    return !causal && keysplit_fits(W, H, nkeys, cus, true) ? lr::ROUTE_KEYSPLIT : lr::ROUTE_STREAM;
+    return !causal && keysplit_images(W, H, nkeys, cus) ? lr::ROUTE_KEYSPLIT : lr::ROUTE_STREAM;
 }
 
 size_t split_bytes(int W, int H, int ns) {

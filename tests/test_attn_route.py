@@ -28,6 +28,14 @@ def test_rows_with_a_workspace(W, H, nkeys, want):
     assert route(W, H, nkeys, workspace=True) == want
 
 
+@pytest.mark.parametrize("W,H", [(32, 40), (64, 33), (513, 12), (600, 16), (2048, 16), (1000, 32)])
+def test_split_area_keeps_the_streaming_kernel(W, H):
+    """From 4,096 keys and 33 blocks of 256 queries on, a workspace call runs the streaming kernel with its split tail."""
+    for nkeys in (4096, 8192, 16384):
+        assert route(W, H, nkeys, workspace=True) == STREAM
+    assert route(W, H, 4095, workspace=True) != STREAM
+
+
 @pytest.mark.parametrize("W,p0,want", [(100, 0, PIPE_W4), (448, 0, PIPE_W4), (128, 320, PIPE_W4), (449, 0, KEYSPLIT),
                                        (128, 321, KEYSPLIT)])
 def test_causal_calls_count_the_keys_they_see(W, p0, want):
