@@ -118,8 +118,11 @@ bool keysplit_rows(int W, int H, int all_keys, int causal, int p0, int cus, bool
 // The kernel of a call over key and value rows under LR_ATTN_CFG_AUTO. ranges: the call can be split over the keys
 // (split_count, and its workspace holds the partials); split_area: its workspace holds the streaming kernel's split area;
 // narrow: its strides suit the kernels that take 32-bit per-lane row offsets (wider ones go on to the pipelined kernels).
-// Up to 24 key tiles the key-split kernel is as fast as the split over workgroups and its merge launch (500 queries x 1,100
-// keys x 16 heads 20.7 / 30.0 us, 150 x 1,000 x 32 19.1 / 22.9, 218 x 1,500 x 16 24.4 / 24.6; 2,500 keys 35.0 / 27.3).
+// The split over workgroups against the key-split kernel, from 16 key tiles on (us, split / key-split): the former's time
+// grows with the rows whose partials it writes and merges, the latter's with its steps, whatever the rows (1 query x 16
+// heads x 1,344 keys 13.3 / 25.3, 128 x 16 x 1,216 17.4 / 24.9, 218 x 16 x 961 22.6 / 21.2, 1,100 23.6 / 22.7, 1,216 23.5 /
+// 24.5, 400 x 16 x 961 26.7 / 20.8, 1,344 29.0 / 26.1). A 256-query block of at most 128 rows runs one wave a SIMD, which halves
+// the split's products. So the key-split kernel takes blocks of more rows up to 10 + rows / 512 key tiles, at most 20.
 // With a split area the streaming kernel's tail puts all workgroups on the calls it takes: from 4,096 keys on the key-split
 // kernel is slower on them (streaming / key-split, us, keys and values not in the caches: 32 queries x 40 heads 52 / 98 and 84 /
 // 190 over 4,096 and 8,192 keys, 600 x 16 58 / 84 and 92 / 158, 2,048 x 16 79 / 85 and 134 / 156, 1,000 x 32 over 16,384
@@ -127,7 +130,8 @@ bool keysplit_rows(int W, int H, int all_keys, int causal, int p0, int cus, bool
 int rows_route(int W, int H, int nkeys, int causal, int p0, int cus, bool ranges, bool split_area, bool narrow) {
     const bool stream = stream_rows(W, H, nkeys, causal, split_area, cus);
     const bool keysplit = narrow && !(stream && split_area) && keysplit_rows(W, H, nkeys, causal, p0, cus, split_area);
-    if (ranges && !(keysplit && nkeys <= 24 * 64)) return lr::ROUTE_KEY_RANGES;
+    const int64_t tiles = ((int64_t)nkeys + 63) / 64, rows = (int64_t)W * H;
+    if (ranges && !(keysplit && W > 128 && tiles <= std::min<int64_t>(20, 10 + rows / 512))) return lr::ROUTE_KEY_RANGES;
     if (keysplit) return lr::ROUTE_KEYSPLIT;
     if (stream) return lr::ROUTE_STREAM;
     // 128 queries per workgroup, two workgroups per CU, unless non-causal 256-query blocks fill whole rounds of

@@ -36,6 +36,15 @@ def test_split_area_keeps_the_streaming_kernel(W, H):
     assert route(W, H, 4095, workspace=True) != STREAM
 
 
+@pytest.mark.parametrize("W,H,nkeys,want", [
+    (1, 16, 961, KEY_RANGES), (128, 16, 961, KEY_RANGES), (128, 32, 961, KEY_RANGES),   # one wave a SIMD
+    (218, 8, 961, KEY_RANGES), (218, 16, 1024, KEYSPLIT), (218, 16, 1025, KEY_RANGES),  # 1,744 rows; 3,488: 16 tiles
+    (400, 16, 1280, KEYSPLIT), (400, 16, 1281, KEY_RANGES),                             # 6,400: 20
+    (218, 16, 960, KEYSPLIT)])                                                          # below 16 tiles nothing is split
+def test_split_over_workgroups_or_key_split(W, H, nkeys, want):
+    assert route(W, H, nkeys, workspace=True) == want
+
+
 @pytest.mark.parametrize("W,p0,want", [(100, 0, PIPE_W4), (448, 0, PIPE_W4), (128, 320, PIPE_W4), (449, 0, KEYSPLIT),
                                        (128, 321, KEYSPLIT)])
 def test_causal_calls_count_the_keys_they_see(W, p0, want):
