@@ -93,25 +93,27 @@ bool keysplit_images(int W, int H, int nkeys, int cus) {
     return (T + 1) / 2 <= (tail * T + tail_wg - 1) / tail_wg + 12;
 }
 
-// The same over key and value rows, for calls whose other kernel is a pipelined one (or, without scratch, the streaming
-// kernel's whole blocks): non-causal ones of at most one round of its blocks (600 x 16 heads 14.9 / 16.5 us, 1,024 queries x
-// 1,104 keys x 32 23.6 / 26.5, 1,280 x 24 26.1 / 27.2, and 2,000 x 24, 1.5 rounds, 69.6 / 60.3). The pipelined kernel starts sooner (~2.5 us: fewer loads before its first product, no
-// merge), so calls of fewer than 8 key tiles keep it (320 x 4 heads 11.7 / 10.4 us, 256 x 24 10.6 / 9.8). Causal calls
-// take the key-split kernel whatever their size: its blocks run longest first and each in half the steps (1,500 queries
-// x 1,577 keys, 32 heads over 8, 32.7 / 40.4 us; 2,048 42.7 / 57.8; 4,096 140 / 187; 4,608 x 24 142 / 178).
-// (All taken before the key-split kernel summed its rounded probabilities, which adds 1 to 3 % to its side: 600 x 16 15.8 us,
-// 1,000 queries x 1,500 keys x 24 heads 30.0 / 33.0, 300 x 3,000 x 16 42.8 / 53.5, causal 500 x 16 13.8 / 15.2.)
-// What counts are the keys that some row sees: a causal chunk at the front of a longer key buffer is a short call (64 queries at
-// position 0 x 16 heads 8.0 us by the key-split kernel, 6.8 by the pipelined one; one query 7.3 and 5.7).
-bool keysplit_rows(int W, int H, int all_keys, int causal, int p0, int cus, bool split_area) {
+// Whether a call over key and value rows runs the key-split kernel in place of a pipelined one (or, without scratch, of the
+// streaming kernel's whole blocks). (us, this kernel / the other; keys and values in the L2s unless said otherwise.)
+//  * Non-causal calls of at most one round of its blocks (600 x 16 heads 15.8 / 16.5, 1,024 queries x 1,104 keys x 32 23.6 /
+//    26.5, 1,280 x 24 26.1 / 27.2, 300 x 3,000 x 16 42.8 / 53.5; 2,000 x 24, 1.5 rounds, 69.6 / 60.3).
+//  * Causal calls: its blocks run longest first and each in half the steps (1,500 queries x 1,577 keys, 32 heads over 8, 32.7 /
+//    40.4; 2,048 42.7 / 57.8; 4,096 140 / 187; 4,608 x 24 142 / 178). What counts are the keys that some row sees: a chunk at
+//    the front of a longer key buffer is a short call (64 queries at position 0 x 16 heads 8.0 / 6.8; one query 7.3 / 5.7).
+//  * Not short calls: the pipelined kernel starts ~2.5 us sooner (fewer loads before its first product, no merge). Causal:
+//    from 8 key tiles on. Non-causal: from 10 (256 x 16 heads over 512, 576 and 640 keys 12.9 / 13.2, 14.7 / 14.4 and 14.5 /
+//    15.2; from the 256 MB cache 14.5 / 13.9, 16.2 / 14.9 and 16.1 / 15.7).
+//  * Not at most 64 rows: the pipelined kernel's waves without rows do no products, this one's do (1 and 64 queries x 16 heads x
+//    2,048 keys 28.8 / 31.5 and 29.6 / 33.0, but from the 256 MB cache 34.5 / 34.1 and 35.5 / 35.7 and from memory 46.9 / 38.9
+//    and 47.7 / 40.0).
+bool keysplit_rows(int W, int H, int all_keys, int causal, int p0, int cus) {
     const int nkeys = causal ? (int)std::min<int64_t>(all_keys, (int64_t)p0 + W) : all_keys;
-    if (nkeys <= 7 * 64 || cus < 1) return false;
+    if (W <= 64 || nkeys <= (causal ? 7 : 9) * 64 || cus < 1) return false;
     const int64_t blocks = (int64_t)((W + 127) / 128) * H;
     if (blocks > 1 << 22) return false;   // (a grid's work-items are counted in 32 bits)
     // few workgroups over many keys wait for memory, not for each other: two tiles in flight a workgroup are then no
-    // better than the pipelined kernel's ring (64 queries x 32 heads, 4,096 / 32,768 keys 68 / 713 us against 64 / 635;
-    // 128 x 4 heads, 8,192 / 16,384 keys 102 / 243 against 123 / 239; 500 x 16 heads, 32,768 keys 475 against 483)
-    if ((causal || !split_area) && nkeys >= 4096 && (W <= 64 || (nkeys >= 16384 && blocks <= 32))) return false;
+    // better than the pipelined kernel's ring (500 queries x 16 heads, 32,768 keys 475 us against 483)
+    if (nkeys >= 16384 && blocks <= 32) return false;
     return causal || blocks <= cus;
 }
 
@@ -129,7 +131,7 @@ bool keysplit_rows(int W, int H, int all_keys, int causal, int p0, int cus, bool
 // 244 / 327).
 int rows_route(int W, int H, int nkeys, int causal, int p0, int cus, bool ranges, bool split_area, bool narrow) {
     const bool stream = stream_rows(W, H, nkeys, causal, split_area, cus);
-    const bool keysplit = narrow && !(stream && split_area) && keysplit_rows(W, H, nkeys, causal, p0, cus, split_area);
+    const bool keysplit = narrow && !(stream && split_area) && keysplit_rows(W, H, nkeys, causal, p0, cus);
     const int64_t tiles = ((int64_t)nkeys + 63) / 64, rows = (int64_t)W * H;
     if (ranges && !(keysplit && W > 128 && tiles <= std::min<int64_t>(20, 10 + rows / 512))) return lr::ROUTE_KEY_RANGES;
     if (keysplit) return lr::ROUTE_KEYSPLIT;

@@ -17,7 +17,7 @@ def test_sizes_no_call_takes():
     (2000, 24, 2000, PIPE_W4),       # 384: past one round
     (16384, 4, 2000, PIPE_W8),       # 256 blocks of 256 queries
     (4608, 24, 4608, STREAM),        # from 4,096 keys on, 432 blocks of 256 queries
-    (320, 24, 320, PIPE_W4),         # too few key tiles for the key-split kernel's longer start
+    (560, 24, 560, PIPE_W4),         # too few key tiles for the key-split kernel's longer start
 ])
 def test_rows(W, H, nkeys, want):
     assert route(W, H, nkeys) == want
@@ -43,6 +43,13 @@ def test_split_area_keeps_the_streaming_kernel(W, H):
     (218, 16, 960, KEYSPLIT)])                                                          # below 16 tiles nothing is split
 def test_split_over_workgroups_or_key_split(W, H, nkeys, want):
     assert route(W, H, nkeys, workspace=True) == want
+
+
+@pytest.mark.parametrize("W,nkeys,causal,want", [
+    (1, 1500, 0, PIPE_W4), (1, 3000, 1, PIPE_W4), (64, 3000, 0, PIPE_W4), (65, 3000, 0, KEYSPLIT), (65, 3000, 1, KEYSPLIT),
+    (128, 576, 0, PIPE_W4), (128, 577, 0, KEYSPLIT), (128, 449, 1, KEYSPLIT), (128, 448, 1, PIPE_W4)])
+def test_few_rows_and_short_calls_keep_the_pipelined_kernel(W, nkeys, causal, want):
+    assert route(W, 16, nkeys, causal=causal, p0=(nkeys - W) * causal) == want
 
 
 @pytest.mark.parametrize("W,p0,want", [(100, 0, PIPE_W4), (448, 0, PIPE_W4), (128, 320, PIPE_W4), (449, 0, KEYSPLIT),
