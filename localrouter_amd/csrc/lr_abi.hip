@@ -100,6 +100,9 @@ bool keysplit_images(int W, int H, int nkeys, int cus) {
 //  * Causal calls: its blocks run longest first and each in half the steps (1,500 queries x 1,577 keys, 32 heads over 8, 32.7 /
 //    40.4; 2,048 42.7 / 57.8; 4,096 140 / 187; 4,608 x 24 142 / 178). What counts are the keys that some row sees: a chunk at
 //    the front of a longer key buffer is a short call (64 queries at position 0 x 16 heads 8.0 / 6.8; one query 7.3 / 5.7).
+//    Not where the chunk is short beside the keys before it, so that all its blocks are about as long, and its blocks are
+//    between one round and two (1,500 queries x 24 heads behind 750, 1,500, 3,000 and 12,000
+//    keys 46.7 / 54.3, 69.7 / 72.6, 114.5 / 108.4 and 380 / 321).
 //  * Not short calls: the pipelined kernel starts ~2.5 us sooner (fewer loads before its first product, no merge). Causal:
 //    from 8 key tiles on. Non-causal: from 10 (256 x 16 heads over 512, 576 and 640 keys 12.9 / 13.2, 14.7 / 14.4 and 14.5 /
 //    15.2; from the 256 MB cache 14.5 / 13.9, 16.2 / 14.9 and 16.1 / 15.7).
@@ -114,7 +117,8 @@ bool keysplit_rows(int W, int H, int all_keys, int causal, int p0, int cus) {
     // few workgroups over many keys wait for memory, not for each other: two tiles in flight a workgroup are then no
     // better than the pipelined kernel's ring (500 queries x 16 heads, 32,768 keys 475 us against 483)
     if (nkeys >= 16384 && blocks <= 32) return false;
-    return causal || blocks <= cus;
+    if (blocks <= cus) return true;
+    return causal && !(blocks <= 2 * (int64_t)cus && 2 * (int64_t)std::min(p0, nkeys) > nkeys);
 }
 
 // The kernel of a call over key and value rows under LR_ATTN_CFG_AUTO. ranges: the call can be split over the keys

@@ -52,6 +52,15 @@ def test_few_rows_and_short_calls_keep_the_pipelined_kernel(W, nkeys, causal, wa
     assert route(W, 16, nkeys, causal=causal, p0=(nkeys - W) * causal) == want
 
 
+@pytest.mark.parametrize("W,p0,want", [
+    (1280, 100000, KEYSPLIT),                               # 240 blocks: one round
+    (1500, 1500, KEYSPLIT), (1500, 1501, PIPE_W4),          # 288, 1.1 rounds: as many keys before the chunk as in it
+    (2688, 30000, PIPE_W4), (2816, 30000, KEYSPLIT)])       # 504 and 528: two rounds
+def test_causal_chunks_behind_many_keys(W, p0, want):
+    """Blocks of about the same length fill whole rounds or lose one, as a non-causal call's."""
+    assert route(W, 24, p0 + W, HK=1, causal=1, p0=p0) == want
+
+
 @pytest.mark.parametrize("W,p0,want", [(100, 0, PIPE_W4), (448, 0, PIPE_W4), (128, 320, PIPE_W4), (449, 0, KEYSPLIT),
                                        (128, 321, KEYSPLIT)])
 def test_causal_calls_count_the_keys_they_see(W, p0, want):
