@@ -442,9 +442,6 @@ __global__ __launch_bounds__(256) void attn_split_combine_kernel(AttnArgs a) {
     float M = m;
 #pragma unroll
     for (int x = 32; x > 0; x >>= 1) M = fmaxf(M, __shfl_xor(M, x, 64));
-    // A range that saw a key counts, whatever its weight underflows to: 0 times an infinity or NaN among its values is NaN,
-    // as in an unsplit call. A range without a sum (no key; or l = NaN, which reaches the row through L) has none to give.
-    const uint64_t seen = __builtin_amdgcn_ballot_w64(m > -INFINITY);
     const float w = m > -INFINITY ? __builtin_amdgcn_exp2f(m - M) : 0.0f;
     float L = w * l;
 #pragma unroll
@@ -454,12 +451,18 @@ __global__ __launch_bounds__(256) void attn_split_combine_kernel(AttnArgs a) {
         float2 v[8];
 #pragma unroll
         for (int j = 0; j < 8; ++j) v[j] = *reinterpret_cast<const float2*>(po + (int64_t)min(s0 + j, ns - 1) * D);
+        // (all of them loaded here: the compiler moved the first one's load behind its condition below, 0.9 us)
+#pragma unroll
+        for (int j = 0; j < 8; ++j) asm volatile("" : "+v"(v[j].x), "+v"(v[j].y));
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
-            const bool take = s0 + j < ns && ((seen >> (s0 + j)) & 1);
-            const float ws = __shfl(w, (s0 + j) & 63, 64);
-            o0 = take ? fmaf(ws, v[j].x, o0) : o0;
-            o1 = take ? fmaf(ws, v[j].y, o1) : o1;
+            // A range that saw a key counts, whatever its weight underflows to: 0 times an infinity or NaN among its values
+            // is NaN, as in an unsplit call. A range without a sum (no key; or l = NaN, which reaches the row through L)
+            // has none to give.
+            const float ms = __shfl(m, s0 + j, 64);
+            const float ws = __builtin_amdgcn_exp2f(ms - M);
+            o0 = ms > -INFINITY ? fmaf(ws, v[j].x, o0) : o0;
+            o1 = ms > -INFINITY ? fmaf(ws, v[j].y, o1) : o1;
         }
     }
     const float inv = 1.0f / L;
