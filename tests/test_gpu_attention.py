@@ -164,16 +164,20 @@ def test_attention_head_major_kv(cfg):
     assert_close(from_dev(out), _ref(q, k, v, causal=True, p0=p0), what=f"head-major cfg{cfg}")
 
 
-@pytest.mark.parametrize("W,nk,H,HK,causal,p0", [(300, 4100, 17, 17, 0, 0), (513, 4097, 12, 6, 0, 0),
-                                                 (700, 999, 3, 1, 1, 299), (64, 4160, 33, 33, 0, 0)])
+@pytest.mark.parametrize("W,nk,H,HK,causal,p0", [(2100, 4100, 17, 17, 0, 0), (2100, 4097, 18, 9, 0, 0),
+                                                 (700, 999, 3, 1, 1, 299), (64, 4160, 257, 257, 0, 0)])
 def test_stream_rows_equal_images(W, nk, H, HK, causal, p0):
     """The streaming kernel over key rows gathers each key tile into the layout of a tile image; over images of the same
     keys (lr_joint_kv_prepare with every key a prefix key: copied unchanged) and the same queries
     (lr_joint_attention_images, which cuts the last partial round of blocks over the workgroups when that pays) the
-    output must be the same bits. Non-causal: lr_attention_bf16_ws, which takes the streaming kernel from 4,096 keys and
-    33 query blocks on (the same split tail, its partials and counters in the caller's workspace); causal (never
-    split): lr_attention_bf16_ex with LR_ATTN_CFG_STREAM_W8."""
+    output must be the same bits. Non-causal (more 128-query blocks than compute units, so that the images take the
+    streaming kernel too): lr_attention_bf16_ws, which takes the streaming kernel from 4,096 keys and 33 query blocks on
+    (the same split tail, its partials and counters in the caller's workspace); causal (never split):
+    lr_attention_bf16_ex with LR_ATTN_CFG_STREAM_W8."""
+    from tests._util import STREAM, route
     print(f"\n[stream rows = images] W={W} nk={nk} H={H} HK={HK} causal={causal}", flush=True)
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    assert route(W, H, nk, HK, causal=causal, p0=p0, images=True, cus=cus) == STREAM
     q, k, v = _qkv(20, W, nk, H, HK)
     dq, dk, dv = to_dev(q), to_dev(k), to_dev(v)
     ws = torch.empty(ops.workspace_bytes(nk, HK), dtype=torch.uint8, device="cuda")
@@ -183,12 +187,18 @@ def test_stream_rows_equal_images(W, nk, H, HK, causal, p0):
         rows = ops.attention(dq, dk, dv, causal=True, p0=p0, config=ops.CFG_STREAM_W8)
     else:
         # a workspace of stale bytes: the call clears the counters it needs
+        assert route(W, H, nk, HK, workspace=True, cus=cus) == STREAM
         assert ops.attention_ws_bytes(W, H, nk, False) == 69207040   # the streaming kernel's split area
         wsr = torch.full((ops.attention_ws_bytes(W, H, nk, False),), 0x5A, dtype=torch.uint8, device="cuda")
         rows = ops.attention_ws(dq, dk, dv, workspace=wsr)
     torch.cuda.synchronize()
     assert torch.equal(rows, img)
-    assert_close(from_dev(rows), _ref(q, k, v, causal=bool(causal), p0=p0), what="stream rows")
+    # the first and last row of every 256-query block, and some between, of every head
+    some = np.unique(np.concatenate([np.arange(0, W, 256), np.minimum(np.arange(255, W + 255, 256), W - 1),
+                                     np.arange(0, W, 97)]))
+    kw = dict(causal=True, p0=p0) if causal else {}
+    ref = oracle.attention(bf16_f32(q), bf16_f32(k), bf16_f32(v), precise=False, rows=some, **kw)
+    assert_close(from_dev(rows)[some], ref, what="stream rows")
 
 
 @pytest.mark.parametrize("W,nk,H,HK", [(6400, 4100, 12, 12), (6400, 4100, 12, 4), (4608, 4096, 24, 24)])

@@ -2,7 +2,7 @@
 over alternating 64-key tiles, merged through LDS. The sizes are those where its cut can go wrong: one query row, the
 edges of a 128-query block, an odd number of key tiles (the second group's last tile is masked whole), a partial last
 tile in either group, one step in all, causal blocks whose second group sees no key, GQA. The calls take it by their
-sizes (LR_ATTN_CFG_AUTO); each is checked against the oracle at the bar of tests/_util.py, and over every stride form
+sizes (LR_ATTN_CFG_AUTO), which every test asserts first; each is checked against the oracle at the bar of tests/_util.py, and over every stride form
 against the pipelined kernel (an explicit configuration) to within two bf16 roundings."""
 from __future__ import annotations
 
@@ -10,7 +10,7 @@ import numpy as np
 import pytest
 
 import oracle
-from tests._util import assert_close, bf16_f32, from_dev, to_dev
+from tests._util import KEYSPLIT, assert_close, bf16_f32, from_dev, route, to_dev
 from tests.test_gpu_attention import _qkv, _ref, _sign_ramp, _sign_ramp_expected
 
 pytestmark = pytest.mark.gpu
@@ -19,16 +19,22 @@ torch = pytest.importorskip("torch")
 from localrouter_amd import _lib, ops  # noqa: E402
 
 
+def _takes_keysplit(W, nk, H, HK, causal=0, p0=0, images=False):
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    assert route(W, H, nk, HK, causal=causal, p0=p0, images=images, cus=cus) == KEYSPLIT
+
+
 @pytest.mark.parametrize("W,nk,H,HK,causal,p0", [
-    (1, 449, 3, 3, 0, 0),        # one row; 8 tiles, the last with one key (second group)
-    (127, 512, 2, 1, 0, 0), (128, 513, 2, 2, 0, 0), (129, 576, 4, 2, 0, 0),
+    (65, 577, 3, 3, 0, 0),       # a wave with one row, one with none; 10 tiles, the last with one key (second group)
+    (127, 640, 2, 1, 0, 0), (128, 641, 2, 2, 0, 0), (129, 704, 4, 2, 0, 0),
     (300, 1000, 5, 5, 0, 0),     # 16 tiles, a partial one last
     (130, 500, 2, 2, 1, 370),    # causal: the diagonal in the last tiles
     (513, 513, 8, 2, 1, 0),      # causal from position 0: first blocks with an empty second group, H a multiple of 8
-    (256, 449, 3, 1, 1, 0),      # queries past the keys see all of them
-    (70, 1200, 7, 7, 1, 77)])
+    (600, 449, 3, 1, 1, 0),      # queries past the keys see all of them
+    (570, 1200, 7, 7, 1, 77)])   # keys past the queries are seen by none
 def test_keysplit_rows(W, nk, H, HK, causal, p0):
     print(f"\n[keysplit rows] W={W} nk={nk} H={H} HK={HK} causal={causal} p0={p0}", flush=True)
+    _takes_keysplit(W, nk, H, HK, causal, p0)
     q, k, v = _qkv(71, W, nk, H, HK)
     dq, dk, dv = to_dev(q), to_dev(k), to_dev(v)
     got = from_dev(ops.attention(dq, dk, dv, causal=bool(causal), p0=p0))
@@ -61,6 +67,7 @@ def test_keysplit_strides_against_the_pipelined_kernel(layout):
     outs = []
     for cfg in (ops.CFG_AUTO, ops.CFG_PIPE_W4):
         for causal, p0 in ((0, 0), (1, 352)):
+            _takes_keysplit(W, nk, H, HK, causal, p0)
             out = torch.zeros(W, H, 136, dtype=torch.bfloat16, device="cuda")   # rows 544 elements apart, 8 of them unused
             _lib.call("lr_attention_bf16_ex", q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), p0, W, H, HK, nk,
                       causal, ops.SCALE_128, q_rs, k_rs, v_rs, H * 136, k_hs, v_hs, cfg,
@@ -79,6 +86,7 @@ def test_keysplit_overflow_reaches_exact_recomputation(rows):
     those of the falling rows do not; queries and outputs in the same rows."""
     Sq, Sk, H = 260, 700, 2
     print(f"\n[keysplit overflow] rows={rows}", flush=True)
+    _takes_keysplit(Sq, Sk, H, H, images=not rows)
     q, k = _sign_ramp(Sq, Sk, H)
     v = oracle.synth_bf16(72, 3, (Sk, H, 128))
     exp = _sign_ramp_expected(q, k, v, 5.0, ops.SCALE_128)
@@ -96,7 +104,8 @@ def test_keysplit_overflow_reaches_exact_recomputation(rows):
 def test_keysplit_one_group_far_above_the_other():
     """Every second key tile scores ~100 (exp2 domain) above the others: one group's result must vanish beside the
     other's, whichever holds the larger scores."""
-    W, nk, H = 64, 640, 2
+    W, nk, H = 96, 640, 2
+    _takes_keysplit(W, nk, H, H)
     q, k, v = _qkv(73, W, nk, H, H)
     kf = bf16_f32(k)
     for odd in (0, 1):
@@ -111,12 +120,13 @@ def test_keysplit_one_group_far_above_the_other():
         assert_close(got, _ref(qb, kb, v), what=f"odd={odd}")
 
 
-@pytest.mark.parametrize("Sq,Sk,H,HK", [(64, 1, 1, 1), (200, 64, 2, 2), (129, 130, 6, 2), (1280, 1280, 24, 24),
+@pytest.mark.parametrize("Sq,Sk,H,HK", [(64, 1, 1, 1), (1, 65, 2, 2), (200, 64, 2, 2), (129, 130, 6, 2), (1280, 1280, 24, 24),
                                         (1000, 3000, 4, 4)])
 def test_keysplit_images_against_the_streaming_kernel(Sq, Sk, H, HK):
     """The fused call at sizes that take the key-split kernel over tile images, against the explicit streaming
     configuration."""
     print(f"\n[keysplit images] Sq={Sq} Sk={Sk} H={H} HK={HK}", flush=True)
+    _takes_keysplit(Sq, Sk, H, HK, images=True)
     q, _, _ = _qkv(74, Sq, 1, H, HK)
     _, k, v = _qkv(75, 1, Sk, H, HK)
     rng = np.random.default_rng(3)
@@ -133,6 +143,8 @@ def test_keysplit_row_of_one_key_is_its_value():
     rounded values, so the one factor left is p * (1 / p) in fp32, far below a bf16 rounding. Over rows the first row of a
     causal call (its second group of waves sees no key), over images a call of one key."""
     W, H = 600, 3
+    _takes_keysplit(W, W, H, H, causal=1)
+    _takes_keysplit(W, 1, H, H, images=True)
     q, k, v = _qkv(76, W, W, H, H)
     dq, dk, dv = to_dev(q), to_dev(k), to_dev(v)
     got = from_dev(ops.attention(dq, dk, dv, causal=True))
@@ -140,3 +152,19 @@ def test_keysplit_row_of_one_key_is_its_value():
     got = from_dev(ops.joint_attention(dq, dk[:1].contiguous(), dv[:1].contiguous(), table_kind=0))
     torch.cuda.synchronize()
     assert np.array_equal(got, np.broadcast_to(from_dev(dv)[:1], got.shape))
+
+
+@pytest.mark.parametrize("W,nk,H,HK", [(300, 4100, 17, 17), (513, 4097, 12, 6), (65, 650, 33, 33), (129, 704, 4, 1)])
+def test_keysplit_rows_equal_images(W, nk, H, HK):
+    """Over key rows the key-split kernel gathers each key tile into the layout of a tile image: the same bits as over images
+    of the same keys (lr_joint_kv_prepare with every key a prefix key: copied unchanged)."""
+    print(f"\n[keysplit rows = images] W={W} nk={nk} H={H} HK={HK}", flush=True)
+    _takes_keysplit(W, nk, H, HK)
+    _takes_keysplit(W, nk, H, HK, images=True)
+    q, k, v = _qkv(77, W, nk, H, HK)
+    dq, dk, dv = to_dev(q), to_dev(k), to_dev(v)
+    ws = torch.empty(ops.workspace_bytes(nk, HK), dtype=torch.uint8, device="cuda")
+    ops.joint_kv_prepare(dk, dv, ws, table_kind=ops.TABLE_NONE, n_pre=nk)
+    img, rows = ops.joint_attention_images(dq, ws, nk, HK), ops.attention(dq, dk, dv)
+    torch.cuda.synchronize()
+    assert torch.equal(rows, img)

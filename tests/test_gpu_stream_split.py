@@ -2,7 +2,9 @@
 last whole round are cut over all workgroups along their key tiles, each piece leaves an fp32 partial (O, m, l), and
 the last piece to arrive merges them in piece order. Shapes are chosen so that cut blocks have 2, 3 and 4 pieces, the
 whole grid is tail (fewer blocks than CUs), GQA and a ragged last key tile; rows of cut blocks are checked against the
-CPU oracle of the reference's chain (tests/_util.py bar). Repeated calls must give identical bits (the merge order
+CPU oracle of the reference's chain (tests/_util.py bar). The fused calls name the streaming configuration, since by their
+sizes some of these would run the key-split kernel; the row calls, which cannot, are of sizes that lead to the streaming
+kernel. Repeated calls must give identical bits (the merge order
 does not depend on which piece arrives last), and overflow inside cut blocks must reach the exact recomputation."""
 from __future__ import annotations
 
@@ -10,7 +12,7 @@ import numpy as np
 import pytest
 
 import oracle
-from tests._util import assert_close, bf16_f32, from_dev, to_dev
+from tests._util import STREAM, assert_close, bf16_f32, from_dev, route, to_dev
 from tests.test_stream_schedule import schedule
 
 pytestmark = pytest.mark.gpu
@@ -37,7 +39,7 @@ def _run(q, k, v, cos, sin, Sq, Sk):
     tq = (torch.from_numpy(np.ascontiguousarray(cos[:Sq])).cuda(), torch.from_numpy(np.ascontiguousarray(sin[:Sq])).cuda())
     tk = (torch.from_numpy(np.ascontiguousarray(cos[:Sk])).cuda(), torch.from_numpy(np.ascontiguousarray(sin[:Sk])).cuda())
     out = ops.joint_attention(to_dev(q), to_dev(k), to_dev(v), table_kind=ops.TABLE_COSSIN_F32, q_table=tq,
-                              k_table=tk, eps=1e-6)
+                              k_table=tk, eps=1e-6, config=ops.CFG_STREAM_W8)
     torch.cuda.synchronize()
     return from_dev(out)
 
@@ -109,7 +111,8 @@ def test_split_overflow_reaches_exact_recomputation():
     q, k = _sign_ramp(Sq, Sk, H)
     v = oracle.synth_bf16(63, 3, (Sk, H, 128))
     w5 = torch.full((128,), 5.0, dtype=torch.float32, device="cuda")
-    out = ops.joint_attention(to_dev(q), to_dev(k), to_dev(v), q_norm=w5, k_norm=w5, table_kind=0, eps=0.0)
+    out = ops.joint_attention(to_dev(q), to_dev(k), to_dev(v), q_norm=w5, k_norm=w5, table_kind=0, eps=0.0,
+                              config=ops.CFG_STREAM_W8)
     torch.cuda.synchronize()
     got = from_dev(out)
     rows = np.arange(0, Sq, 5)
@@ -125,6 +128,7 @@ def test_rows_split_tail_parity(Sq, Sk, H, HK):
     bits."""
     work, pieces, p = schedule(Sq, H, Sk, _cus())
     assert p["nt"] is not None, "the shape must take the split schedule"
+    assert route(Sq, H, Sk, HK, workspace=True, cus=torch.cuda.get_device_properties(0).multi_processor_count) == STREAM
     print(f"\n[rows split] Sq={Sq} Sk={Sk} H={H} HK={HK} cut blocks {len(pieces)}", flush=True)
     q, k, v, _, _ = _case(64, Sq, Sk, H, HK)
     dq, dk, dv = to_dev(q), to_dev(k), to_dev(v)
