@@ -40,8 +40,9 @@ namespace {
 // so the QK^T MFMAs of the next tile hide the exp/max/sum work of the current one, and every load has two tiles of
 // compute to land.
 
-// NW waves of 32 queries each (two waves per SIMD at NW = 8); 64-key tiles in an NS-stage K/V ring.
-template <int NW, int NS>
+// NW waves of 32 queries each (two waves per SIMD at NW = 8); 64-key tiles in an NS-stage K/V ring. EARLY: a step's refills
+// are all issued at its start instead of spread over its slots (refill_early, launch_attention).
+template <int NW, int NS, bool EARLY>
 __global__ __launch_bounds__(NW * 64, 8 / NW) __attribute__((amdgpu_waves_per_eu(2, 2))) void attn_fwd_pipe_kernel(
     AttnArgs a) {
     static_assert(NS >= 2 && NS <= 4, "2- to 4-stage ring");
@@ -130,6 +131,22 @@ __global__ __launch_bounds__(NW * 64, 8 / NW) __attribute__((amdgpu_waves_per_eu
     auto load_k1 = [&](int slot, int j) { dma16(kp[j], kr_lds + 2 * slot * TILE + wdst + 2 * NW * 512 * j); };
     auto load_v1 = [&](int slot, int j) { dma16(vp[j], vr_lds + 2 * slot * TILE + wdst + 2 * NW * 512 * j); };
 
+    // all of step t's refills (EARLY: the pointers are moved behind the loads, out of their way)
+    auto refill_all = [&](int t) {
+        if (t + NS < ntiles) {
+            if constexpr (!EARLY) next_k(t + NS);
+#pragma unroll
+            for (int j = 0; j < LOADS; ++j) load_k1(t % NS, j);
+            if constexpr (EARLY) next_k(t + NS + 1);
+        }
+        if (t + NS - 1 < ntiles) {
+            if constexpr (!EARLY) next_v(t + NS - 1);
+#pragma unroll
+            for (int j = 0; j < LOADS; ++j) load_v1((t + NS - 1) % NS, j);
+            if constexpr (EARLY) next_v(t + NS);
+        }
+    };
+
     // ---- queries (B operands of S^T = K Q^T), one set per 32-query block
     // ---- prologue loads: K(0 .. NS-1) and V(0 .. NS-2) into the ring first, so that their latency overlaps the
     // query loads (the query's own waits, issued after, are conservative for the ring loads: older loads finish first)
@@ -142,6 +159,10 @@ __global__ __launch_bounds__(NW * 64, 8 / NW) __attribute__((amdgpu_waves_per_eu
         next_v(i);
 #pragma unroll
         for (int j = 0; j < LOADS; ++j) load_v1(i, j);
+    }
+    if constexpr (EARLY) {
+        next_k(NS);
+        next_v(NS - 1);
     }
     bf16x8 qf[NQB][8];
 #pragma unroll
@@ -181,16 +202,7 @@ __global__ __launch_bounds__(NW * 64, 8 / NW) __attribute__((amdgpu_waves_per_eu
         block_barrier();
         for (int t = 0; t < ntiles; ++t) {
             const bool refilled = t + NS < ntiles;
-            if (refilled) {
-                next_k(t + NS);
-#pragma unroll
-                for (int j = 0; j < LOADS; ++j) load_k1(t % NS, j);
-            }
-            if (t + NS - 1 < ntiles) {
-                next_v(t + NS - 1);
-#pragma unroll
-                for (int j = 0; j < LOADS; ++j) load_v1((t + NS - 1) % NS, j);
-            }
+            refill_all(t);
             if (NS == 2 || !refilled) LR_WAIT_VMCNT(0);
             else LR_WAIT_VMCNT((NS - 2) * 2 * LOADS);
             block_barrier();
@@ -292,8 +304,12 @@ __global__ __launch_bounds__(NW * 64, 8 / NW) __attribute__((amdgpu_waves_per_eu
         // 1 KB load a slot below (all of them here held the wave's issue up behind the memory pipe: 3,000 queries x 700 keys
         // x 32 heads 49.0 -> 44.5 us with 128-query workgroups, 3,000 x 3,000 x 24 146.7 -> 139.4)
         const bool refilled = t + NS < ntiles, refill_v = t + NS - 1 < ntiles;
-        if (refilled) next_k(t + NS);
-        if (refill_v) next_v(t + NS - 1);
+        if constexpr (EARLY) {
+            refill_all(t);
+        } else {
+            if (refilled) next_k(t + NS);
+            if (refill_v) next_v(t + NS - 1);
+        }
         {
             // Explicit schedule of the tile's 32 MFMA slots (one wave's instruction stream; a sched_barrier closes
             // every slot, so the compiler keeps each slot's work in it):
@@ -330,7 +346,8 @@ __global__ __launch_bounds__(NW * 64, 8 / NW) __attribute__((amdgpu_waves_per_eu
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
             for (int s = 0; s < 32; ++s) {
-                if (s < LOADS) {
+                if (EARLY) {
+                } else if (s < LOADS) {
                     if (refilled) load_k1(t % NS, s);
                 } else if (s < 2 * LOADS) {
                     if (refill_v) load_v1((t + NS - 1) % NS, s - LOADS);
@@ -469,13 +486,13 @@ __global__ __launch_bounds__(256) void attn_split_combine_kernel(AttnArgs a) {
     *reinterpret_cast<uint32_t*>(a.out + (int64_t)qrow * a.o_rs + head * D + 2 * lane) = pack_bf16x2(o0 * inv, o1 * inv);
 }
 
-template <int NW, int NS>
+template <int NW, int NS, bool EARLY = false>
 hipError_t launch_pipe(const AttnArgs& a, hipStream_t stream) {
     constexpr int BM = 32 * NW;
     const int64_t nqb = (a.W + BM - 1) / BM;
     const int64_t blocks = nqb * a.H * (a.nsplit > 1 ? a.nsplit : 1);
     if (blocks > 0x7fffffff) return hipErrorInvalidValue;
-    hipLaunchKernelGGL((attn_fwd_pipe_kernel<NW, NS>), dim3((unsigned)blocks), dim3(NW * 64), 0, stream, a);
+    hipLaunchKernelGGL((attn_fwd_pipe_kernel<NW, NS, EARLY>), dim3((unsigned)blocks), dim3(NW * 64), 0, stream, a);
     return hipGetLastError();
 }
 
@@ -493,7 +510,8 @@ hipError_t launch_attention(const AttnArgs& a, int config, hipStream_t stream) {
     switch (config) {
         case ATTN_CFG_AUTO:
         case ATTN_CFG_PIPE_W8: return launch_pipe<8, 3>(a, stream);
-        case ATTN_CFG_PIPE_W4: return launch_pipe<4, 2>(a, stream);   // 64 KB of LDS: two per CU
+        case ATTN_CFG_PIPE_W4:   // 64 KB of LDS: two per CU
+            return a.refill_early ? launch_pipe<4, 2, true>(a, stream) : launch_pipe<4, 2>(a, stream);
         default: return hipErrorInvalidValue;
     }
 }

@@ -93,6 +93,15 @@ bool keysplit_images(int W, int H, int nkeys, int cus) {
     return (T + 1) / 2 <= (tail * T + tail_wg - 1) / tail_wg + 12;
 }
 
+// Keys and values that the call's rows see beyond the device's 256 MB cache: every call reads them from memory, and a call of
+// few blocks then waits for its loads, not for its products. How soon a step's loads are issued is what counts (us, refills
+// at the step's start / spread over its slots / key-split kernel, whose tiles come one step ahead: 16 heads x 61,035 keys, 128
+// queries 1,036 / 1,127 / 1,220, 256 1,002 / 1,109 / 1,158, 1,000 961 / 1,086 / 1,087).
+bool beyond_cache(int W, int HK, int nkeys, int causal, int p0) {
+    const int64_t seen = causal ? std::min<int64_t>(nkeys, (int64_t)p0 + W) : nkeys;
+    return seen * HK * (2 * lr::D * 2) > (int64_t)256 << 20;
+}
+
 // Whether a call over key and value rows runs the key-split kernel in place of a pipelined one (or, without scratch, of the
 // streaming kernel's whole blocks). (us, this kernel / the other; keys and values in the L2s unless said otherwise.)
 //  * Non-causal calls of at most one round of its blocks (600 x 16 heads 15.8 / 16.5, 1,024 queries x 1,104 keys x 32 23.6 /
@@ -114,8 +123,8 @@ bool keysplit_rows(int W, int H, int all_keys, int causal, int p0, int cus) {
     if (W <= 64 || nkeys <= (causal ? 7 : 9) * 64 || cus < 1) return false;
     const int64_t blocks = (int64_t)((W + 127) / 128) * H;
     if (blocks > 1 << 22) return false;   // (a grid's work-items are counted in 32 bits)
-    // few workgroups over many keys wait for memory, not for each other: two tiles in flight a workgroup are then no
-    // better than the pipelined kernel's ring (500 queries x 16 heads, 32,768 keys 475 us against 483)
+    // few workgroups over many keys wait for memory, not for each other (1 head, 2,015 queries x 28,107 keys 369 / 410, from
+    // memory 467 / 428)
     if (nkeys >= 16384 && blocks <= 32) return false;
     if (blocks <= cus) return true;
     return causal && !(blocks <= 2 * (int64_t)cus && 2 * (int64_t)std::min(p0, nkeys) > nkeys);
@@ -133,9 +142,10 @@ bool keysplit_rows(int W, int H, int all_keys, int causal, int p0, int cus) {
 // kernel is slower on them (streaming / key-split, us, keys and values not in the caches: 32 queries x 40 heads 52 / 98 and 84 /
 // 190 over 4,096 and 8,192 keys, 600 x 16 58 / 84 and 92 / 158, 2,048 x 16 79 / 85 and 134 / 156, 1,000 x 32 over 16,384
 // 244 / 327).
-int rows_route(int W, int H, int nkeys, int causal, int p0, int cus, bool ranges, bool split_area, bool narrow) {
+int rows_route(int W, int H, int HK, int nkeys, int causal, int p0, int cus, bool ranges, bool split_area, bool narrow) {
     const bool stream = stream_rows(W, H, nkeys, causal, split_area, cus);
-    const bool keysplit = narrow && !(stream && split_area) && keysplit_rows(W, H, nkeys, causal, p0, cus);
+    const bool keysplit = narrow && !(stream && split_area) && keysplit_rows(W, H, nkeys, causal, p0, cus) &&
+                          (stream || !beyond_cache(W, HK, nkeys, causal, p0));
     const int64_t tiles = ((int64_t)nkeys + 63) / 64, rows = (int64_t)W * H;
     if (ranges && !(keysplit && W > 128 && tiles <= std::min<int64_t>(20, 10 + rows / 512))) return lr::ROUTE_KEY_RANGES;
     if (keysplit) return lr::ROUTE_KEYSPLIT;
@@ -182,13 +192,13 @@ int attention_impl(const void* q, const void* k, const void* v, void* out, int p
     a.W = W; a.H = H; a.HK = HK; a.G = H / HK; a.nkeys = nkeys; a.p0 = p0; a.causal = causal;
     a.c = scale * 1.4426950408889634f;
     const int ns = split_count(W, H, nkeys, causal);
-    const int cus = config == LR_ATTN_CFG_AUTO || config == LR_ATTN_CFG_STREAM_W8 ? device_cus() : 0;
+    const int cus = device_cus();
     const bool ws_split_area = workspace && ws_bytes >= (size_t)LR_JOINT_SPLIT_BYTES && aligned(workspace, 256);
     const bool ranges = workspace && ns > 1 && k_hs == lr::D && v_hs == lr::D && ws_bytes >= split_bytes(W, H, ns) &&
                         aligned(workspace, 256);
     const bool narrow = k_rs <= lr::STREAM_MAX_V_RS && v_rs <= lr::STREAM_MAX_V_RS;
     int route = config;
-    if (config == LR_ATTN_CFG_AUTO) route = rows_route(W, H, nkeys, causal, p0, cus, ranges, ws_split_area, narrow);
+    if (config == LR_ATTN_CFG_AUTO) route = rows_route(W, H, HK, nkeys, causal, p0, cus, ranges, ws_split_area, narrow);
     else if (config == LR_ATTN_CFG_PIPE_W8 && ranges) route = lr::ROUTE_KEY_RANGES;
     if (route == lr::ROUTE_KEY_RANGES) {
         a.nsplit = ns;
@@ -212,6 +222,7 @@ int attention_impl(const void* q, const void* k, const void* v, void* out, int p
         }
         return (int)lr::launch_stream(a, nwg, stream, true);
     }
+    a.refill_early = beyond_cache(W, HK, nkeys, causal, p0) && (int64_t)((W + 127) / 128) * H <= cus;
     return (int)lr::launch_attention(a, route, stream);
 }
 
@@ -628,7 +639,7 @@ int lr_attention_route(int W, int H, int HK, int nkeys, int causal, int p0, size
     if (W < 1 || H < 1 || HK < 1 || nkeys < 1 || p0 < 0) return 0;
     if (images) return images_route(W, H, nkeys, causal, std::min(cus, lr::STREAM_MAX_WG));
     const int ns = split_count(W, H, nkeys, causal);
-    return rows_route(W, H, nkeys, causal, p0, cus, ns > 1 && workspace_bytes >= split_bytes(W, H, ns),
+    return rows_route(W, H, HK, nkeys, causal, p0, cus, ns > 1 && workspace_bytes >= split_bytes(W, H, ns),
                       workspace_bytes >= (size_t)LR_JOINT_SPLIT_BYTES, true);
 }
 

@@ -28,6 +28,8 @@ struct AttnArgs {
     int split, tail_wg;
     void* part;
     int* cnt;
+    // Pipelined kernel, 128-query blocks: 1 = a step's refills all at its start
+    int refill_early;
     // Key-split kernel: floor(2^32 / d) (2^32 - 1 for d = 1) for its query blocks a head, H and G. Set by launch_keysplit.
     uint32_t rcp_nqb, rcp_h, rcp_g;
 };

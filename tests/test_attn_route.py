@@ -61,6 +61,20 @@ def test_causal_chunks_behind_many_keys(W, p0, want):
     assert route(W, 24, p0 + W, HK=1, causal=1, p0=p0) == want
 
 
+@pytest.mark.parametrize("W,H,HK,causal", [(300, 16, 16, 0), (500, 32, 32, 1), (1500, 24, 24, 1),
+                                             (1000, 64, 8, 1)])
+def test_keys_beyond_the_cache_keep_the_pipelined_kernel(W, H, HK, causal):
+    """512 bytes a key and key head: 256 MB are 2^19 of them."""
+    last = (1 << 19) // HK
+    assert route(W, H, last + 64, HK, causal, p0=last + 64 - W) == PIPE_W4
+    assert route(W, H, last, HK, causal, p0=last - W) == (KEYSPLIT if (W + 127) // 128 * H <= 256 else PIPE_W4)
+
+
+def test_keys_beyond_the_cache_without_scratch():
+    """Past half a round of 256-query blocks the other kernel is the streaming one's whole blocks: the key-split kernel."""
+    assert route(1000, 32, 50000) == KEYSPLIT and route(1000, 24, 50000) == PIPE_W4
+
+
 @pytest.mark.parametrize("W,p0,want", [(100, 0, PIPE_W4), (448, 0, PIPE_W4), (128, 320, PIPE_W4), (449, 0, KEYSPLIT),
                                        (128, 321, KEYSPLIT)])
 def test_causal_calls_count_the_keys_they_see(W, p0, want):

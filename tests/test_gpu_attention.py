@@ -544,3 +544,22 @@ def test_prepared_rejects_plain_configs():
     for cfg in (ops.CFG_PIPE_W8, ops.CFG_PIPE_W4, 3, 8):
         with pytest.raises(Exception):
             ops.joint_attention_prepared(q, ws, Sk, HK, table_kind=ops.TABLE_NONE, config=cfg)
+
+
+@pytest.mark.parametrize("W,nk,H,causal", [(1, 8200, 64, 0), (100, 8257, 64, 0), (129, 32833, 16, 0), (256, 16500, 32, 1)])
+def test_keys_beyond_the_cache(W, nk, H, causal):
+    """Calls of few blocks over more than 256 MB of keys and values take the 128-query pipelined kernel with a step's
+    refills all at its start: the same bits as the 256-query one's, whose rows go through the same operations in the same
+    order; the last tile partial or whole, a wave without rows, a partly filled block, the causal diagonal."""
+    from tests._util import PIPE_W4, route
+    print(f"\n[beyond the cache] W={W} nk={nk} H={H} causal={causal}", flush=True)
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    p0 = (nk - W) * causal
+    assert H * nk * 512 > 256 << 20 and route(W, H, nk, causal=causal, p0=p0, cus=cus) == PIPE_W4
+    g = torch.Generator(device="cuda")
+    g.manual_seed(nk)
+    q, k, v = (torch.randn(n, H, 128, generator=g, device="cuda").to(torch.bfloat16) for n in (W, nk, nk))
+    auto, w8 = (ops.attention(q, k, v, causal=bool(causal), p0=p0, config=c) for c in (ops.CFG_AUTO, ops.CFG_PIPE_W8))
+    torch.cuda.synchronize()
+    assert torch.isfinite(auto.float()).all()
+    assert torch.equal(auto, w8)
