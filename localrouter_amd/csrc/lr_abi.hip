@@ -78,10 +78,11 @@ bool stream_rows_split(int W, int H, int nkeys, int cus) {
 
 // Whether a non-causal call over tile images runs the key-split kernel (attn_keysplit.hip: 128-query blocks, one workgroup
 // each, two key groups) in place of the streaming kernel: its blocks fit one round of the CUs and, where the streaming
-// kernel would cut its tail, half the key tiles are no more than the tiles a workgroup of that tail takes plus 12 (the
-// ~16 us its partials, merges and longer start cost, at ~1.3 us a tile).
+// kernel would cut its tail, half the key tiles are no more than the tiles a workgroup of that tail takes plus 8 (the
+// ~10 us its partials, merges and longer start cost, at ~1.3 us a tile: 4 heads, 3,300 queries over 3,300 keys, 26 against 18
+// + 8, 53.1 / 54.6; over 3,500, 28 against 19 + 8, 57.0 / 56.2; 4,200 x 4,400 69.6 / 66.2).
 // Measured (us, this kernel / the other): 320 x 4 heads 14.9 / 24.5, 512 x 24 18.8 / 30.9, 1,280 x 24 34.3 / 48.4,
-// 3,000 x 4 43.0 / 50.1; past one round it gains nothing (1,600 x 24, 1.2 rounds, 59.9 / 60.5; 3,000 x 12, 1.1
+// 2,600 x 4 44.2 / 46.7; past one round it gains nothing (1,600 x 24, 1.2 rounds, 59.9 / 60.5; 3,000 x 12, 1.1
 // rounds, 90.8 / 77.5; 4,608 x 24 263 / 248).
 bool keysplit_images(int W, int H, int nkeys, int cus) {
     const int64_t blocks = (int64_t)((W + 127) / 128) * H, T = (nkeys + 63) / 64;
@@ -90,7 +91,7 @@ bool keysplit_images(int W, int H, int nkeys, int cus) {
     const int nwg = std::min(cus, lr::STREAM_MAX_WG);
     if (!lr::stream_split_params(W, H, nkeys, 0, nwg, &tail_wg)) return true;
     const int64_t tail = (int64_t)((W + 255) / 256) * H % nwg;   // <= blocks <= cus: all of them when below nwg
-    return (T + 1) / 2 <= (tail * T + tail_wg - 1) / tail_wg + 12;
+    return (T + 1) / 2 <= (tail * T + tail_wg - 1) / tail_wg + 8;
 }
 
 // Keys and values that the call's rows see beyond the device's 256 MB cache: every call reads them from memory, and a call of

@@ -88,3 +88,9 @@ def test_causal_calls_count_the_keys_they_see(W, p0, want):
 def test_images(Sq, H, Sk, want):
     assert route(Sq, H, Sk, images=True) == want
     assert route(Sq, H, Sk, images=True, causal=1) == STREAM
+
+
+@pytest.mark.parametrize("Sq,Sk,want", [(3300, 3300, KEYSPLIT), (3300, 3500, STREAM), (4200, 4200, STREAM), (100, 2000, KEYSPLIT),
+                                        (100, 5000, STREAM)])
+def test_images_beside_the_split_tail(Sq, Sk, want):
+    assert route(Sq, 4, Sk, images=True) == want
