@@ -197,7 +197,9 @@ int attention_impl(const void* q, const void* k, const void* v, void* out, int p
     const bool ws_split_area = workspace && ws_bytes >= (size_t)LR_JOINT_SPLIT_BYTES && aligned(workspace, 256);
     const bool ranges = workspace && ns > 1 && k_hs == lr::D && v_hs == lr::D && ws_bytes >= split_bytes(W, H, ns) &&
                         aligned(workspace, 256);
-    const bool narrow = k_rs <= lr::STREAM_MAX_V_RS && v_rs <= lr::STREAM_MAX_V_RS;
+    // (the output stride: the streaming kernel's limit. The key-split kernel has none, but would then take calls that are refused
+    // where the streaming kernel is theirs)
+    const bool narrow = k_rs <= lr::STREAM_MAX_V_RS && v_rs <= lr::STREAM_MAX_V_RS && o_rs < ((int64_t)1 << 23);
     int route = config;
     if (config == LR_ATTN_CFG_AUTO) route = rows_route(W, H, HK, nkeys, causal, p0, cus, ranges, ws_split_area, narrow);
     else if (config == LR_ATTN_CFG_PIPE_W8 && ranges) route = lr::ROUTE_KEY_RANGES;

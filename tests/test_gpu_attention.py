@@ -232,6 +232,31 @@ def test_attention_deterministic():
     assert np.array_equal(a, b)
 
 
+@pytest.mark.parametrize("nk,ok", [(4160, False), (1000, True)])
+def test_output_stride_of_2_23_elements(nk, ok):
+    """An output row stride of 2^23 elements or more at sizes of the key-split kernel: refused where the rules' next kernel is the
+    streaming one (from 4,096 keys and half a round of 256-query blocks on), run by the pipelined kernel below."""
+    from localrouter_amd import _lib
+    from tests._util import KEYSPLIT, route
+    W, H, HK = 66, 128, 1
+    print(f"\n[output stride] nk={nk}", flush=True)
+    assert route(W, H, nk, HK, cus=torch.cuda.get_device_properties(0).multi_processor_count) == KEYSPLIT
+    q, k, v = _qkv(24, W, nk, H, HK)
+    dq, dk, dv = to_dev(q), to_dev(k), to_dev(v)
+    rs = 1 << 23
+    out = torch.empty((W - 1) * rs + H * 128, dtype=torch.bfloat16, device="cuda")
+    args = (dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), out.data_ptr(), 0, W, H, HK, nk, 0, ops.SCALE_128, H * 128, HK * 128,
+            rs, torch.cuda.current_stream().cuda_stream)
+    if not ok:
+        assert _lib.load().lr_attention_bf16(*args) == 1
+        return
+    _lib.call("lr_attention_bf16", *args)
+    want = ops.attention(dq, dk, dv, config=ops.CFG_PIPE_W4)
+    torch.cuda.synchronize()
+    got = out.as_strided((W, H * 128), (rs, 1))
+    assert torch.equal(got, want.view(W, H * 128))
+
+
 def test_attention_rejects_bad_args():
     """Rejected arguments return hipErrorInvalidValue and launch nothing."""
     from localrouter_amd import _lib
