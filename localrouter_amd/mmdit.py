@@ -10,7 +10,7 @@ from __future__ import annotations
 import ctypes
 from pathlib import Path
 
-from . import _lib, ops
+from . import _lib
 
 HEADER = Path(__file__).resolve().parent.parent / "include" / "lr_mmdit.h"
 
@@ -154,6 +154,8 @@ class MMDiTBlock:
 
     def __call__(self, txt, img, t, cos, sin, stream=None):
         import torch
+
+        from . import ops
         n_txt, n_img = txt.shape[0], img.shape[0]
         assert txt.dtype == img.dtype == torch.bfloat16 and txt.is_contiguous() and img.is_contiguous()
         assert t.dtype == torch.float32 and cos.dtype == sin.dtype == torch.float32

@@ -232,6 +232,17 @@ def test_ops_has_no_cpu_path():
         ops.attention(q, q, q)
 
 
+@pytest.mark.parametrize("module", ["localrouter_amd", "localrouter_amd._lib", "localrouter_amd.mmdit", "localrouter_amd.rope",
+                                    "localrouter_amd.rope_host"])
+def test_modules_load_without_torch(module):
+    """Only ops needs torch to be imported: the bindings' declarations and the table builders load without it."""
+    import subprocess
+    import sys
+    code = f"import sys; sys.modules['torch'] = None; sys.path.insert(0, {str(_lib.PKG.parent)!r}); import {module}"
+    r = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True)
+    assert r.returncode == 0, r.stderr
+
+
 def test_mmdit_abi_on_cpu():
     """include/lr_mmdit.h: exports, workspace sizes and argument rejection (no GPU call is reached)."""
     import ctypes
