@@ -588,3 +588,13 @@ def test_keys_beyond_the_cache(W, nk, H, causal):
     torch.cuda.synchronize()
     assert torch.isfinite(auto.float()).all()
     assert torch.equal(auto, w8)
+
+
+def test_stream_handle_is_the_current_stream():
+    """ops takes the current stream's raw handle from torch's binding: the number torch.cuda.current_stream() gives, on the
+    default stream, inside a stream context and after it."""
+    side = torch.cuda.Stream()
+    assert ops._stream() == torch.cuda.current_stream().cuda_stream
+    with torch.cuda.stream(side):
+        assert ops._stream() == torch.cuda.current_stream().cuda_stream == side.cuda_stream
+    assert ops._stream() == torch.cuda.current_stream().cuda_stream != side.cuda_stream
