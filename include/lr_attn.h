@@ -63,10 +63,13 @@ typedef struct ihipStream_t* lr_stream_t;
 
 /* Attention tile configurations for the _ex entry points. 0 = the library's choice by the call's sizes:
  *   fused and prepared calls: LR_ATTN_CFG_STREAM_W8, or, non-causal with few 128-query blocks (at most one per compute
- *     unit), the key-split kernel over the same tile images (attn_keysplit.hip: 128 queries per workgroup, two groups of
- *     waves over alternating key tiles);
- *   attention over key and value rows, from 449 keys on: the key-split kernel for causal calls and for non-causal ones
- *     of at most one 128-query block per compute unit; else LR_ATTN_CFG_STREAM_W8 for non-causal calls of at least
+ *     unit) and not too many key tiles, the key-split kernel over the same tile images (attn_keysplit.hip: 128 queries per
+ *     workgroup, two groups of waves over alternating key tiles);
+ *   attention over key and value rows: the key-split kernel for calls of more than 64 queries, causal ones from 449 keys
+ *     that a query sees on (not for a chunk behind more keys than its own where its blocks are between one and two per
+ *     compute unit), non-causal ones from 577 keys on and of at most one 128-query block per compute unit, neither over
+ *     more keys and values than the device's cache holds (256 MB) nor with strides beyond LR_ATTN_CFG_STREAM_W8's; else
+ *     LR_ATTN_CFG_STREAM_W8 for non-causal calls of at least
  *     4,096 keys whose 256-query blocks fill at least half a round of the device's compute units without leaving a last
  *     round less than half full, or fill two rounds or more; other calls LR_ATTN_CFG_PIPE_W4, or LR_ATTN_CFG_PIPE_W8 when
  *     non-causal and the 256-query blocks fill whole rounds of the compute units. The workspace call
@@ -114,16 +117,16 @@ int lr_attention_bf16_ex(const void* q, const void* k, const void* v, void* out,
                          int config, lr_stream_t stream);
 
 /*
- * lr_attention_bf16 with device scratch. A non-causal call with at most 32 blocks of 256 queries x heads and more than
- * 1,536 keys (24 tiles of 64; e.g. 218 queries over 50,220 keys), or at least 961 where the key-split kernel does not
- * cover the call, is split over the keys into ranges that fill the GPU, each range's partial result written to the
- * workspace, then merged (flash-decoding). Other non-causal calls of at least
- * 4,096 keys (but for those of few query blocks whose keys the key-split kernel covers sooner) run
+ * lr_attention_bf16 with device scratch. A non-causal call with at most 32 blocks of 256 queries x heads and at least 961
+ * keys (16 tiles of 64; e.g. 218 queries over 50,220 keys) is split over the keys into ranges that fill the GPU, each range's
+ * partial result written to the workspace, then merged (flash-decoding); up to 20 tiles, with more than 128 queries and many
+ * rows, it runs the key-split kernel instead. Other non-causal calls of at least 4,096 keys run
  * LR_ATTN_CFG_STREAM_W8 over the key rows, whose last partial round of query blocks is cut over all workgroups
  * along the keys, the pieces' partials and arrival counters in the workspace (LR_JOINT_SPLIT_BYTES; the call clears
- * the counters itself). Every other call runs as lr_attention_bf16. lr_attention_ws_bytes is the workspace the call
- * needs (0: none; workspace may then be NULL); those bytes must not overlap q, k, v or out (rejected). Results equal
- * lr_attention_bf16's to fp32 rounding. Calls that overlap on one workspace race.
+ * the counters itself). Every other call runs as lr_attention_bf16. lr_attention_ws_bytes is the workspace that the call
+ * asks for by its sizes (0: none; workspace may then be NULL): an upper bound, as a call that runs the key-split kernel
+ * leaves it unused; those bytes must not overlap q, k, v or out (rejected). Results equal
+ * lr_attention_bf16's to the rounding of the probabilities to bf16 and fp32 sums. Calls that overlap on one workspace race.
  */
 size_t lr_attention_ws_bytes(int W, int H, int nkeys, int causal);
 int lr_attention_bf16_ws(const void* q, const void* k, const void* v, void* out, int p0, int W, int H, int HK,
@@ -137,7 +140,8 @@ int lr_attention_bf16_ws(const void* q, const void* k, const void* v, void* out,
  * [W][H*128], k, v rows [nkeys][HK*128] (kv_row_stride for both). kmask: device u8 [nkeys]; n_valid: the number of
  * nonzero bytes, known on the host as the engine's `valid` (1 <= n_valid <= nkeys). The kept keys and value rows are
  * gathered into the workspace, then attended as lr_attention_bf16 does; the workspace's first
- * lr_attention_kmask_workspace_bytes bytes must not overlap kmask, q, k, v or out (rejected). kmask = NULL: no mask
+ * lr_attention_kmask_workspace_bytes bytes (4 a kept key, reserved, then the gathered rows) must not overlap kmask, q, k, v
+ * or out (rejected). kmask = NULL: no mask
  * (n_valid = nkeys, no workspace needed).
  */
 size_t lr_attention_kmask_workspace_bytes(int n_valid, int HK);

@@ -32,11 +32,12 @@ inline bool rows_ok(const void* p, int64_t rs, int heads) {
 
 inline bool scale_ok(float s) { return s > 0.0f && isfinite(s); }
 
-// Key-split count for plain attention over value rows (the pipelined kernel, 256-query blocks): a non-causal launch
+// Count of key ranges for plain attention over value rows (the pipelined kernel, 256-query blocks): a non-causal launch
 // with at most 32 query blocks and at least 16 key tiles is split over the keys into enough ranges of at least 4 key
 // tiles to give ~256 workgroups, then merged by a combine pass. 1 = no split (causal calls are never split). Measured
 // at 218 queries x 16 / 24 heads the split takes 0.77 / 0.47 / 0.22 of the 128-query pipelined kernel's time at
-// 2,000 / 8,000 / 50,220 keys and 1.34 at 600 keys; at 600-1,280 queries the streaming kernel's split tail is faster.
+// 2,000 / 8,000 / 50,220 keys and 1.34 at 600 keys; at 600-1,280 queries the streaming kernel's split tail is faster (and
+// rows_route has the calls that the key-split kernel takes from it).
 int split_count(int W, int H, int nkeys, int causal) {
     if (causal || W < 1 || H < 1 || nkeys < 1) return 1;
     const int64_t blocks = (int64_t)((W + 255) / 256) * H;
@@ -48,8 +49,8 @@ int split_count(int W, int H, int nkeys, int causal) {
     return (tiles + per - 1) / per;   // no empty range
 }
 
-// Whether a non-causal call over key and value rows that is not key-split runs the streaming kernel (reading key rows
-// into tile images in LDS) instead of the pipelined kernels. Measured from 218 to 50,220 queries x 4-32 heads: below
+// Whether a non-causal call over key and value rows that is not split over the keys runs the streaming kernel (reading key
+// rows into tile images in LDS) instead of the pipelined kernels. Measured from 218 to 50,220 queries x 4-32 heads: below
 // 4,096 keys the 128-query pipelined kernel is as fast or faster. From 4,096 keys on, with a workspace (its split tail
 // cutting the last partial round of blocks over the workgroups) the streaming kernel takes 0.55-0.93 of the pipelined
 // kernel's time from 33 query blocks on. Without one it runs whole 256-query blocks (a last partial pass shared by
@@ -251,7 +252,7 @@ static_assert(lr::STREAM_PART_BYTES + lr::STREAM_CNT_BYTES == (int64_t)LR_JOINT_
 size_t ws_bytes_needed(int Sk, int HK) { return 2 * (size_t)lr::img_bytes(Sk, HK) + LR_JOINT_SPLIT_BYTES; }
 inline char* split_area(void* ws, int Sk, int HK) { return static_cast<char*>(ws) + 2 * lr::img_bytes(Sk, HK); }
 
-// the configurations of the fused and prepared calls (both the streaming kernel)
+// the configurations of the fused and prepared calls (images_route, and the streaming kernel by name)
 inline bool is_stream(int config) { return config == LR_ATTN_CFG_AUTO || config == LR_ATTN_CFG_STREAM_W8; }
 
 // compute units of the current device: the streaming kernel's grid (one workgroup per CU); queried on every call,
@@ -404,8 +405,8 @@ bool images_stage_ok(const void* q_prep, int64_t p_rs, const void* ws, size_t ws
     return !overlap(so, rows_span(q_prep, Sq, p_rs, H)) && !overlap(rows_span(q_prep, Sq, p_rs, H), ws_span(ws, Sk, HK));
 }
 
-// The attention stage (arguments checked): the persistent streaming kernel, one workgroup per CU (at most
-// STREAM_MAX_WG), its last partial round of query blocks cut over all of them (partials and counters in the
+// The attention stage (arguments checked): the key-split kernel where images_route says so, else the persistent streaming
+// kernel, one workgroup per CU (at most STREAM_MAX_WG), its last partial round of query blocks cut over all of them (partials and counters in the
 // workspace's split area). v / v_rs: the value rows it reads (the caller's, or null for the workspace's value area).
 int images_launch(const void* q_prep, int64_t p_rs, const void* ws, void* out, int64_t o_rs, int Sq, int Sk, int H,
                   int HK, int p0, int causal, float scale, hipStream_t stream, const void* v = nullptr,
@@ -696,9 +697,9 @@ int lr_attention_bf16_ws(const void* q, const void* k, const void* v, void* out,
 
 size_t lr_attention_kmask_workspace_bytes(int n_valid, int HK) {
     if (n_valid < 1 || HK < 1) return 0;
-    const size_t idx = ((size_t)n_valid * 4 + 255) & ~(size_t)255;
+    const size_t reserved = ((size_t)n_valid * 4 + 255) & ~(size_t)255;   // unused: callers size their buffers by it
     const size_t rows = (((size_t)n_valid * HK * lr::D * 2) + 255) & ~(size_t)255;
-    return idx + 2 * rows;
+    return reserved + 2 * rows;
 }
 
 int lr_attention_kmask_bf16(const void* q, const void* k, const void* v, void* out, const void* kmask, int n_valid,
@@ -717,7 +718,7 @@ int lr_attention_kmask_bf16(const void* q, const void* k, const void* v, void* o
     if (W < 1 || H < 1 || HK < 1 || H % HK != 0 || !scale_ok(scale) || !rows_ok(q, q_row_stride, H) ||
         !rows_ok(out, out_row_stride, H) || W > INT_MAX - 512 || nkeys > INT_MAX - 512)
         return ERR_ARGS;
-    // the compaction writes the kept keys' indices, keys and values to the workspace while it reads kmask, k and v,
+    // the compaction writes the kept keys and values to the workspace while it reads kmask, k and v,
     // and the attention then reads them beside q and writes out: the workspace's bytes overlap none of those
     {
         const uintptr_t lo = reinterpret_cast<uintptr_t>(workspace), mk = reinterpret_cast<uintptr_t>(kmask);
@@ -728,10 +729,10 @@ int lr_attention_kmask_bf16(const void* q, const void* k, const void* v, void* o
             return ERR_ARGS;
     }
     char* ws = static_cast<char*>(workspace);
-    const size_t idx_bytes = ((size_t)n_valid * 4 + 255) & ~(size_t)255;
+    const size_t reserved = ((size_t)n_valid * 4 + 255) & ~(size_t)255;
     const size_t rows = (((size_t)n_valid * HK * lr::D * 2) + 255) & ~(size_t)255;
-    void* kc = ws + idx_bytes;
-    void* vc = ws + idx_bytes + rows;
+    void* kc = ws + reserved;
+    void* vc = ws + reserved + rows;
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
     const hipError_t e = lr::launch_compact_keys(k, v, kv_row_stride, static_cast<const uint8_t*>(kmask), nkeys,
                                                  n_valid, HK, kc, vc, s);
