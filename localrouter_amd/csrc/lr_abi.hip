@@ -406,8 +406,9 @@ bool images_stage_ok(const void* q_prep, int64_t p_rs, const void* ws, size_t ws
 }
 
 // The attention stage (arguments checked): the key-split kernel where images_route says so, else the persistent streaming
-// kernel, one workgroup per CU (at most STREAM_MAX_WG), its last partial round of query blocks cut over all of them (partials and counters in the
-// workspace's split area). v / v_rs: the value rows it reads (the caller's, or null for the workspace's value area).
+// kernel, one workgroup per CU (at most STREAM_MAX_WG), its last partial round of query blocks cut over all of them
+// (partials and counters in the workspace's split area). v / v_rs: the value rows it reads (the caller's, or null for the
+// workspace's value area).
 int images_launch(const void* q_prep, int64_t p_rs, const void* ws, void* out, int64_t o_rs, int Sq, int Sk, int H,
                   int HK, int p0, int causal, float scale, hipStream_t stream, const void* v = nullptr,
                   int64_t v_rs = 0, int config = LR_ATTN_CFG_AUTO) {
